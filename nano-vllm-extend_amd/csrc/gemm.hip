@@ -13,16 +13,23 @@
 // k values of one row of each operand, so every operand read is one 16-byte
 // LDS read.
 //
-// Tiling: a workgroup of 4 waves (one per SIMD, one workgroup per CU)
-// computes a BM x 256 tile of C (BM = 256, or 192 where that fills the last
-// wave of tiles better; 64 x 128 or 64 x 64, several workgroups per CU, for
-// small M, with three or four LDS stages when K is long: gemm_tn_deep_kernel
-// below), K in steps of 64.  Wave (wm, wn) owns rows BM / 2 wm
-// .. and columns 128 wn ..: BM / 64 x 4 accumulator tiles of 32 x 32 (256
-// registers at BM = 256, kept in AGPRs), 64 products per step.
+// Four kernels, chosen by gemm_launch:
+//   gemm_tn_pp_kernel    256 x 256 tiles, the last few as 128 x 128 quarters;
+//                        8 waves in two alternating groups, persistent (most
+//                        shapes with more than a few hundred rows)
+//   gemm_tn_deep_kernel  64 x 128 or 64 x 64, three or four LDS stages (a
+//                        decode in_proj)
+//   gemm_tn_kernel       the general one: 256 x 256 or 192 x 256 where K is an
+//                        odd multiple of 64, 64-row tiles where K is short
 //
-// Operand path: global -> LDS directly (buffer_load ... lds, no registers),
-// two stages of BM + 256 rows x 128 bytes (128 KiB at BM = 256).  The loads
+// gemm_tn_kernel: a workgroup of 4 waves (one per SIMD, one workgroup per CU)
+// computes a BM x BN tile of C, K in steps of 64.  Wave (wm, wn) owns rows BM /
+// 2 wm .. and columns BN / 2 wn ..: BM / 64 x BN / 64 accumulator tiles of 32 x
+// 32 (256 registers at 256 x 256, kept in AGPRs), 64 products per step.
+//
+// Operand path (all kernels): global -> LDS directly (buffer_load ... lds, no
+// registers).  gemm_tn_kernel has two stages of BM + BN rows x 128 bytes (128
+// KiB at 256 x 256).  The loads
 // of step s + 1 are spread one per product over the first half of step s (a
 // burst stalls the waves on the shared address unit).  Operand fragments
 // are read one 16-deep sub-step ahead of their products, interleaved one read
@@ -45,6 +52,8 @@
 // (bf16) and g = -exp(A_log) softplus(a + dt_bias) (fp32) are written from the
 // bf16-rounded values with the gate kernel's arithmetic (gdn::gate_beta,
 // gdn::gate_g), so they equal gdn_g_beta applied to C.
+#include <algorithm>
+
 #include "gdn_common.h"
 
 namespace {
@@ -369,6 +378,373 @@ __global__ __launch_bounds__(kGemmThreads, kMinWG) void gemm_tn_kernel(const uin
   gemm_store<BM, BN>(acc, out, M, N, m0, n0, wave, lane, gt, nk % 2 ? st0 : st1);
 }
 
+// ---- 16 rows x 32 columns of accumulators to the output (the 8-wave kernel) ----
+// Lane (lr, lg) holds C[row0 + lr][cb + 8 lg .. + 7] in c0 (the first four) and
+// c1: one 16-byte piece, four lanes filling 64 contiguous bytes of a row.
+__device__ __forceinline__ void gemm_store16(const gdn::f32x4_t& c0, const gdn::f32x4_t& c1, const GemmOut& out,
+                                             int M, int N, int row0, int cb, int lane, const GemmGates& gt,
+                                             uint16_t* gs) {
+  const int lr = lane & 15, lg = lane >> 4;
+  if (cb >= N || row0 >= M) return;  // wave-uniform
+  auto pick = [](int t, auto a0, auto a1, auto a2, auto a3) { return t == 0 ? a0 : t == 1 ? a1 : t == 2 ? a2 : a3; };
+  const uint4 w = make_uint4(gdn::f2bf2(c0[0], c0[1]), gdn::f2bf2(c0[2], c0[3]), gdn::f2bf2(c1[0], c1[1]),
+                             gdn::f2bf2(c1[2], c1[3]));
+  // the part of the block's first 16 columns (wave-uniform)
+  const int s = cb < out.end[0] ? 0 : cb < out.end[1] ? 1 : cb < out.end[2] ? 2 : 3;
+  const int cend = pick(s, out.end[0], out.end[1], out.end[2], out.end[3]);
+  const int m = row0 + lr, n = cb + 8 * lg;
+  if (pick(s, out.vec[0], out.vec[1], out.vec[2], out.vec[3]) && cb + 32 <= cend) {
+    // the whole block in one part with 16-byte rows
+    uint16_t* c = pick(s, out.c[0], out.c[1], out.c[2], out.c[3]) - pick(s, 0, out.end[0], out.end[1], out.end[2]);
+    const int64_t ld = pick(s, out.ld[0], out.ld[1], out.ld[2], out.ld[3]);
+    if (m < M) *reinterpret_cast<uint4*>(c + m * ld + n) = w;
+  } else if (m < M) {
+    // a part boundary inside the block, the last columns, or rows without
+    // 16-byte alignment
+    const int sp = n >= cend && cend < N ? s + 1 : s;
+    const int pe = pick(sp, out.end[0], out.end[1], out.end[2], out.end[3]);
+    const int pb = pick(sp, 0, out.end[0], out.end[1], out.end[2]);
+    uint16_t* crow = pick(sp, out.c[0], out.c[1], out.c[2], out.c[3]) +
+                     static_cast<int64_t>(m) * pick(sp, out.ld[0], out.ld[1], out.ld[2], out.ld[3]) - pb;
+    if (pick(sp, out.vec[0], out.vec[1], out.vec[2], out.vec[3]) && n + 8 <= pe) {
+      *reinterpret_cast<uint4*>(crow + n) = w;
+    } else {
+      const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+        if (n + t < pe) crow[n + t] = static_cast<uint16_t>(ww[t / 2] >> (16 * (t % 2)));
+    }
+  }
+  // gate outputs from the bf16-rounded b and a columns of this block, through
+  // the wave's own 1 KiB of LDS (see gemm_store)
+  if (gt.g && cb + 32 > gt.gate_col && cb < gt.gate_col + 2 * gt.Hv) {
+    *reinterpret_cast<uint4*>(gs + 32 * lr + 8 * lg) = w;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+#pragma unroll 1
+    for (int e = lane; e < 16 * 32; e += 64) {
+      const int r = e >> 5, c = e & 31;
+      const int mm = row0 + r, nn = cb + c, col = nn - gt.gate_col;
+      if (mm >= M || nn >= N || col < 0 || col >= 2 * gt.Hv) continue;
+      const float v = gdn::bf2f(gs[32 * r + c]);
+      if (col < gt.Hv) {
+        gt.beta[static_cast<int64_t>(mm) * gt.Hv + col] = gdn::gate_beta(v);
+      } else {
+        const int h = col - gt.Hv;
+        gt.g[static_cast<int64_t>(mm) * gt.Hv + h] =
+            gdn::gate_g(v, gdn::load_param(gt.A_log, h, gt.param_f32), gdn::load_param(gt.dt_bias, h, gt.param_f32));
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// ---- 256 x 256 tiles, 8 waves in two alternating groups ----
+// What bounds it: the matrix cores at the clock that the power limit leaves
+// (8192^3: busy 0.83-0.87 of the cycles at 1.6 GHz).
+//
+// Two waves per SIMD, one of each group (wave w and w + 4: row halves wm = 0
+// and 1).  A K-step of 64 is two load sections (12 LDS fragment reads, 4 loads
+// into LDS, a wait) and two product sections (32 products of 16 x 16 x 32: 512
+// cycles) per wave, separated by workgroup barriers; group 1 runs one section
+// behind group 0, so on each SIMD one wave multiplies while the other reads and
+// loads, and neither the address unit nor an LDS wait holds up the products, as
+// they do with one wave per SIMD (gemm_tn_kernel).  Sections of 16 products (4
+// load sections per step) were slower: 16384 x 12352 x 2048 651 -> 646 us with
+// the longer ones, 8192^3 774 -> 757.  Products of 16 x 16 x 32 move half the
+// accumulator bytes per operation of 32 x 32 x 16 ones, which the power limit
+// turns into clock: 653 -> 613 us and 768 -> 704 us.
+//
+// LDS: half tiles of 128 rows x 64 values (16 KiB), two of A, two of B, two
+// stages; eight objects, so that the compiler's load counting sees which reads
+// wait for which loads.  A section loads into the two half tiles that the
+// section before it read (both groups are done with them: group 1's reads of
+// that section ended before the barrier that started this one), so every load
+// has three sections (1,500 cycles and more) to land; the wait at a section's
+// end leaves the newest two sections' loads (8) in flight.  The reads of a
+// section are: row half 0 of A, column half 1 of B; then row half 1 of A and
+// column half 0 of B of the next step (the other column half stays in
+// registers).
+//
+// Persistent: one workgroup per CU walks its tiles, and the loads run on into
+// the next tile's first steps, in flight during the stores of this one.  The
+// tiles past the last full round of 256 (up to 128 of them) run as quarters of
+// 128 x 128 over all CUs: 12.25 rounds cost 12.4 and not 13 (16384 x 12352 x
+// 2048: 611 -> 593 us; 2.09 rounds, 17001 x 2048 x 2048: 135 -> 116).
+//
+// Columns: B's rows are read in the order 8 (j / 4) + 4 t + j % 4 (fragment row
+// j of column tile t), so that a lane's two accumulators of a tile pair are 8
+// consecutive columns of a row and the stores need no lane exchange; B's LDS
+// swizzle follows that order (swb_off).
+//
+// Against the one-wave-per-SIMD kernel, same box: 16384 x 12352 x 2048 760 ->
+// 593 us (1.40 PFLOP/s), 16384 x 2048 x 4096 206 -> 185, 17001 x 8224 x 2048
+// 508 -> 425, 1949 x 12352 x 2048 100 -> 87, 1949 x 2048 x 4096 42.6 -> 38.
+constexpr int kPPThreads = 512;
+
+__device__ __forceinline__ void half_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+
+// s_waitcnt vmcnt(8) lgkmcnt(0): all but the newest 8 loads have landed and
+// every LDS read has returned
+constexpr int kWaitPP = 8 | (7 << 4);
+
+// LDS offset of granule c of row r in a half tile of B (see the column order
+// below)
+__device__ __forceinline__ int swb_off(int r, int c) {
+  return r * 128 + ((c ^ (((r >> 1) & 1) | (((r >> 3) & 3) << 1))) << 4);
+}
+
+// grid = 8 * min(32, ...) workgroups of 512; tiles 0 .. whole - 1 run as 256 x
+// 256, the rest as quarters.  K is a multiple of 128.
+__global__ __launch_bounds__(kPPThreads, 2) void gemm_tn_pp_kernel(const uint16_t* __restrict__ A, int64_t lda,
+                                                                  const uint16_t* __restrict__ B, int64_t ldb,
+                                                                  GemmOut out, int M, int N, int K, GemmGates gt,
+                                                                  int whole) {
+  constexpr int kHalf = 128 * 128;  // bytes of a half tile: 128 rows of 64 values
+  __shared__ __align__(16) uint8_t a00[kHalf];
+  __shared__ __align__(16) uint8_t a01[kHalf];
+  __shared__ __align__(16) uint8_t a10[kHalf];
+  __shared__ __align__(16) uint8_t a11[kHalf];
+  __shared__ __align__(16) uint8_t b00[kHalf];
+  __shared__ __align__(16) uint8_t b01[kHalf];
+  __shared__ __align__(16) uint8_t b10[kHalf];
+  __shared__ __align__(16) uint8_t b11[kHalf];
+  __shared__ __align__(16) uint16_t gscr[8][16 * 32];
+
+  const int mb_n = (M + 255) / 256, nb_n = (N + 255) / 256;
+  // XCD x (workgroups b % 8 == x) walks a contiguous range of the tiles
+  const int xcd = blockIdx.x % gdn::kNumXcd, slot = blockIdx.x / gdn::kNumXcd, stride = gridDim.x / gdn::kNumXcd;
+  const int tiles = mb_n * nb_n;
+  const int per_xcd = (whole + gdn::kNumXcd - 1) / gdn::kNumXcd;
+  const int xend = min((xcd + 1) * per_xcd, whole);
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const int lr = lane & 15, lg = lane >> 4;
+
+  auto tile_of = [&](int t, int& m0, int& n0) {
+    const int per_group = kGroupM * nb_n;
+    const int grp = t / per_group, in_grp = t % per_group;
+    const int gm = min(kGroupM, mb_n - grp * kGroupM);
+    m0 = 256 * (grp * kGroupM + in_grp % gm);
+    n0 = 256 * (in_grp / gm);
+  };
+  // the wave's loads: 1 KiB blocks w and w + 8 of each half tile
+  const __amdgpu_buffer_rsrc_t ra = rsrc_of(A), rb = rsrc_of(B);
+  const int ldrow = 8 * wave + (lane >> 3);
+  const int gcol_a = 8 * ((lane & 7) ^ (((wave & 1) << 2) | (lane >> 4)));
+  const int gcol_b = 8 * ((lane & 7) ^ (((wave & 3) << 1) | ((lane >> 4) & 1)));
+  int va[2][2], vb[2][2];
+  auto set_offsets = [&](int m0, int n0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        va[h][i] = static_cast<int>((min(m0 + 128 * h + 64 * i + ldrow, M - 1) * lda + gcol_a) * 2);
+        vb[h][i] = static_cast<int>((min(n0 + 128 * h + 64 * i + ldrow, N - 1) * ldb + gcol_b) * 2);
+      }
+  };
+  auto dma = [&](const __amdgpu_buffer_rsrc_t& r, uint8_t* dst, const int (&v)[2], int kbyte) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dma16(r, dst + (wave + 8 * i) * 1024, v[i], kbyte);
+  };
+  typedef gdn::s16x8_t frag_t;
+  auto read_a = [&](const uint8_t* h, frag_t (&f)[4][2]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        f[i][ks] = *reinterpret_cast<const frag_t*>(h + sw_off(64 * wm + 16 * i + lr, 4 * ks + lg));
+  };
+  auto read_b = [&](const uint8_t* h, frag_t (&f)[2][2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        f[t][ks] = *reinterpret_cast<const frag_t*>(h + swb_off(32 * wn + 8 * (lr >> 2) + 4 * t + (lr & 3), 4 * ks + lg));
+  };
+  gdn::f32x4_t acc[2][2][4][2];  // [row half][column half][16-row tile][column tile]
+  // one row half of A against both column halves of B
+  auto prod = [&](gdn::f32x4_t (&c0)[4][2], gdn::f32x4_t (&c1)[4][2], const frag_t (&fa)[4][2],
+                  const frag_t (&f0)[2][2], const frag_t (&f1)[2][2]) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) c0[i][t] = gdn::mfma16x16x32(f0[t][ks], fa[i][ks], c0[i][t]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) c1[i][t] = gdn::mfma16x16x32(f1[t][ks], fa[i][ks], c1[i][t]);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    half_barrier();
+  };
+  auto mem_end = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(kWaitPP);
+    half_barrier();
+  };
+  const int nk = K / kBK;  // even
+  int L = xcd * per_xcd + slot;
+  if (L < xend) {
+  int m0, n0;
+  tile_of(L, m0, n0);
+  set_offsets(m0, n0);
+  dma(rb, b00, vb[0], 0);
+  dma(ra, a00, va[0], 0);
+  dma(rb, b01, vb[1], 0);
+  dma(rb, b10, vb[0], 128);
+  dma(ra, a01, va[1], 0);
+  dma(ra, a10, va[0], 128);
+  dma(rb, b11, vb[1], 128);
+  frag_t fa[4][2], fb0[2][2], fb1[2][2], fbn[2][2];
+  __builtin_amdgcn_s_waitcnt(12 | (7 << 4));
+  half_barrier();
+  read_b(b00, fb0);
+  mem_end();
+  for (;;) {
+    const int Ln = L + stride;
+    const int m0c = m0, n0c = n0;
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) acc[a][b][i][t] = gdn::f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (wm) half_barrier();
+    int kb = 256;
+    for (int s = 0; s < nk; s += 2) {
+      const int ka = kb - 128;  // of step s + 1: the current tile's
+      int v1[2] = {va[1][0], va[1][1]};
+      if (s + 2 == nk) {
+        // the next loads are the next tile's first steps (past the last tile
+        // they repeat this one's)
+        if (Ln < xend) {
+          tile_of(Ln, m0, n0);
+          set_offsets(m0, n0);
+        }
+        kb = 0;
+      }
+      dma(rb, b00, vb[0], kb);
+      dma(ra, a11, v1, ka);
+      read_a(a00, fa);
+      read_b(b01, fb1);
+      mem_end();
+      prod(acc[0][0], acc[0][1], fa, fb0, fb1);
+      dma(ra, a00, va[0], kb);
+      dma(rb, b01, vb[1], kb);
+      read_a(a01, fa);
+      read_b(b10, fbn);
+      mem_end();
+      prod(acc[1][0], acc[1][1], fa, fb0, fb1);
+      dma(rb, b10, vb[0], kb + 128);
+      dma(ra, a01, va[1], kb);
+      read_a(a10, fa);
+      read_b(b11, fb1);
+      mem_end();
+      prod(acc[0][0], acc[0][1], fa, fbn, fb1);
+      dma(ra, a10, va[0], kb + 128);
+      dma(rb, b11, vb[1], kb + 128);
+      read_a(a11, fa);
+      read_b(b00, fb0);
+      mem_end();
+      prod(acc[1][0], acc[1][1], fa, fbn, fb1);
+      kb += 256;
+    }
+    if (!wm) half_barrier();
+    // (the lane from an opaque copy, so that no address of the epilogue is
+    // kept in registers across the loop)
+    int tid_e = static_cast<int>(threadIdx.x);
+    asm volatile("" : "+v"(tid_e));
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          gemm_store16(acc[a][b][i][0], acc[a][b][i][1], out, M, N, m0c + 128 * a + 64 * wm + 16 * i,
+                       n0c + 128 * b + 32 * wn, tid_e & 63, gt, gscr[wave]);
+    if (Ln >= xend) break;
+    L = Ln;
+  }
+  }
+  // The tiles after the whole ones, as quarters of 128 x 128: per K-step one
+  // half tile of A and one of B, so the eight LDS objects hold four steps.
+  const int nq = 4 * (tiles - whole);
+  const int q_xcd = (nq + gdn::kNumXcd - 1) / gdn::kNumXcd;
+  const int qend = min((xcd + 1) * q_xcd, nq);
+  for (int q = xcd * q_xcd + slot; q < qend; q += stride) {
+    int m0, n0;
+    tile_of(whole + (q >> 2), m0, n0);
+    m0 += 128 * ((q >> 1) & 1);
+    n0 += 128 * (q & 1);
+    if (m0 >= M || n0 >= N) continue;  // (the whole workgroup)
+    set_offsets(m0, n0);
+    __builtin_amdgcn_s_waitcnt(7 << 4);  // loads into the stages, of a tile before
+    half_barrier();
+    auto load = [&](uint8_t* a, uint8_t* b, int step) {
+      const int kb = 128 * min(step, nk - 1);
+      dma(ra, a, va[0], kb);
+      dma(rb, b, vb[0], kb);
+    };
+    load(a00, b00, 0);
+    load(a01, b01, 1);
+    load(a10, b10, 2);
+    gdn::f32x4_t c[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) c[i][t] = gdn::f32x4_t{0.f, 0.f, 0.f, 0.f};
+    frag_t fa[4][2], fb[2][2];
+    // step s from (a, b); the loads of step s + 3 into (an, bn)
+    auto step = [&](const uint8_t* a, const uint8_t* b, uint8_t* an, uint8_t* bn, int s) {
+      load(an, bn, s + 3);
+      read_a(a, fa);
+      read_b(b, fb);
+      mem_end();
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) c[i][t] = gdn::mfma16x16x32(fb[t][ks], fa[i][ks], c[i][t]);
+      __builtin_amdgcn_s_setprio(0);
+      half_barrier();
+    };
+    __builtin_amdgcn_s_waitcnt(kWaitPP);  // step 0
+    half_barrier();
+    if (wm) half_barrier();
+    for (int s = 0; s < nk; s += 4) {
+      step(a00, b00, a11, b11, s);
+      step(a01, b01, a00, b00, s + 1);
+      if (s + 2 >= nk) break;
+      step(a10, b10, a01, b01, s + 2);
+      step(a11, b11, a10, b10, s + 3);
+    }
+    if (!wm) half_barrier();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      gemm_store16(c[i][0], c[i][1], out, M, N, m0 + 64 * wm + 16 * i, n0 + 32 * wn, lane, gt, gscr[wave]);
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+}
+
 // ---- small M (decode batches): a deeper load pipeline ----
 // gemm_tn_kernel's two stages let a step's loads arrive during one step's
 // products, which at 64-row tiles are four to eight products: every step then
@@ -512,40 +888,59 @@ namespace {
 // entry points).
 int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, const GemmOut& out, int M, int N,
                 int K, const GemmGates& gt, void* stream) {
-  // Tile: 256 x 256 with one workgroup per CU, so a launch runs in
-  // ceil(tiles / CUs) waves of tiles, each taking time in proportion to the
-  // tile's rows.  192 x 256 is taken when its waves x rows is smaller (a
-  // short last wave of 256-row tiles, e.g. 536 tiles = 2.09 waves -> 712 =
-  // 2.78).  When 256 x 256 tiles would not fill half of the CUs (small M:
-  // decode batches), 64 x 128 tiles, two or more workgroups per CU, spread
-  // the work over the whole chip; 64 x 64 when even those would not.
   const int64_t nb256 = (N + 255) / 256;
   const int64_t t256 = ((M + 255) / 256) * nb256, t192 = ((M + 191) / 192) * nb256;
-  const int64_t w256 = (t256 + kCUs - 1) / kCUs, w192 = (t192 + kCUs - 1) / kCUs;
-  const int64_t t64x128 = ((M + 63) / 64) * ((N + 127) / 128);
-  const int cfg = t256 >= kCUs / 2 ? (w192 * 192 < w256 * 256 ? 1 : 0) : t64x128 >= kCUs / 2 ? 2 : 3;
-  const int64_t tiles = cfg == 3 ? ((M + 63) / 64) * ((N + 63) / 64) : cfg == 2 ? t64x128 : cfg == 1 ? t192 : t256;
-  const int64_t grid = gdn::kNumXcd * ((tiles + gdn::kNumXcd - 1) / gdn::kNumXcd);
+  const int64_t t128 = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128);
+  const int64_t t64x128 = static_cast<int64_t>((M + 63) / 64) * ((N + 127) / 128);
+  const int64_t t64 = static_cast<int64_t>((M + 63) / 64) * ((N + 63) / 64);
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 g3(static_cast<unsigned>(grid)), b3(kGemmThreads);
-  // The 64-row tiles take the deeper load pipeline when K has at least 16
-  // steps (graph-replayed launches, 256 x 8224 x 2048: 21.1 -> 19.0 us; 256
-  // x 2048 x 2048: 10.1 -> 9.3 us; 64 x 8224 x 2048: 17.2 -> 10.0 us); with
-  // fewer its prologue and the repeated last loads cost more than it saves
-  // (1000 x 2080 x 512: 6.5 -> 7.0 us).
+  auto grid = [](int64_t wgs) {
+    return dim3(static_cast<unsigned>(gdn::kNumXcd * ((wgs + gdn::kNumXcd - 1) / gdn::kNumXcd)));
+  };
+  const dim3 b3(kGemmThreads);
+  // 256 x 256 tiles when they fill half of the CUs, or quarters of them when
+  // those make one round that fills more than half (1949 x 2048 x 4096: 42.6
+  // -> 37.7 us against 64 x 128 tiles, 900 x 4096 x 2048 23.9 -> 22.4, 256 x
+  // 8224 x 2048 20.1 -> 19.8; two rounds of quarters do not pay, 400 x 12352 x
+  // 2048: 35.0 -> 38.1).  The two-stage loop takes K in pairs of steps.
+  const bool wide = t256 >= kCUs / 2;
+  if (K % (2 * kBK) == 0 && (wide || (t128 > kCUs / 2 && t128 <= kCUs))) {
+    const int64_t rem = t256 % kCUs;
+    const int64_t whole = rem <= kCUs / 2 ? t256 - rem : t256;
+    const int64_t wgs = std::min<int64_t>(kCUs, std::max(whole, 4 * (t256 - whole)));
+    gemm_tn_pp_kernel<<<grid(wgs), dim3(kPPThreads), 0, st>>>(A, lda, B, ldb, out, M, N, K, gt,
+                                                              static_cast<int>(whole));
+    return gdn_launch_status();
+  }
+  if (wide) {
+    // Odd multiples of 64: a launch runs in ceil(tiles / CUs) waves of tiles,
+    // each taking time in proportion to the tile's rows; 192 x 256 is taken when
+    // its waves x rows is smaller (a short last wave of 256-row tiles, e.g. 536
+    // tiles = 2.09 waves -> 712 = 2.78).
+    const int64_t w256 = (t256 + kCUs - 1) / kCUs, w192 = (t192 + kCUs - 1) / kCUs;
+    if (w192 * 192 < w256 * 256)
+      gemm_tn_kernel<192, 256, 1><<<grid(t192), b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+    else
+      gemm_tn_kernel<256, 256, 1><<<grid(t256), b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+    return gdn_launch_status();
+  }
+  // Small M.  The deeper load pipelines pay when K has at least 16 steps (with
+  // fewer their prologue and the repeated last loads cost more than they save:
+  // 1000 x 2080 x 512: 6.5 -> 7.0 us).
   const bool deep = K / kBK >= 16;
-  if (cfg == 3 && deep)
-    gemm_tn_deep_kernel<64, 4><<<g3, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
-  else if (cfg == 3)
-    gemm_tn_kernel<64, 64, 2><<<g3, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
-  else if (cfg == 2 && deep)
-    gemm_tn_deep_kernel<128, 3><<<g3, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
-  else if (cfg == 2)
-    gemm_tn_kernel<64, 128, 2><<<g3, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
-  else if (cfg == 1)
-    gemm_tn_kernel<192, 256, 1><<<g3, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
-  else
-    gemm_tn_kernel<256, 256, 1><<<g3, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+  // 64 x 128 tiles, two or more workgroups per CU, spread the work over the
+  // whole chip; 64 x 64 when even those would not.
+  if (t64x128 >= kCUs / 2) {
+    if (deep)
+      gemm_tn_deep_kernel<128, 3><<<grid(t64x128), b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+    else
+      gemm_tn_kernel<64, 128, 2><<<grid(t64x128), b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+  } else {
+    if (deep)
+      gemm_tn_deep_kernel<64, 4><<<grid(t64), b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+    else
+      gemm_tn_kernel<64, 64, 2><<<grid(t64), b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+  }
   return gdn_launch_status();
 }
 

@@ -53,6 +53,36 @@ def test_gemm_against_fp32_matmul(pkg, dev, M, N, K):
     _check(c, ref, sc, f"gemm {M}x{N}x{K}")
 
 
+# The 8-wave kernel's quarters alone (128 x 128; K of 2, 4 and 6 steps, ragged
+# rows and columns, an empty quarter past M), behind whole tiles, and whole tiles
+# of an uneven last round; its K restriction (192: gemm_tn_kernel at 256 and 192
+# rows).  Hv > 0: the columns go to four parts with gate outputs
+# (b and a the last 2 Hv columns).
+@pytest.mark.parametrize("M,N,K,Hv", [(1949, 2048, 128, 0), (1100, 4000, 256, 16), (1153, 2072, 384, 4),
+                                      (4100, 4008, 384, 4), (4500, 3000, 256, 0), (8190, 2047, 192, 0),
+                                      (17000, 2048, 192, 0)])
+def test_gemm_kernel_edges(pkg, dev, M, N, K, Hv):
+    gen = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=gen).to(BF16)
+    w = (torch.randn(N, K, generator=gen) / math.sqrt(K)).to(BF16)
+    if not Hv:
+        c = pkg.ops.linear(a.to(dev), w.to(dev))
+        _check(c, *_ref(a, w), f"gemm {M}x{N}x{K}")
+        return
+    A_log = (torch.rand(Hv, generator=gen) * math.log(16)).to(dev)
+    dt_bias = (torch.rand(Hv, generator=gen) * 2 - 1).to(dev)
+    first = (N - 2 * Hv) // 32 * 16
+    widths = [first, N - 2 * Hv - first, Hv, Hv] if Hv % 16 == 0 else [first, 32, N - first - 32]
+    parts, g, beta = pkg.ops.linear_cols(a.to(dev), w.to(dev), widths,
+                                         gates={"gate_col": N - 2 * Hv, "A_log": A_log, "dt_bias": dt_bias})
+    c = torch.cat(parts, 1)
+    _check(c, *_ref(a, w), f"gemm parts {M}x{N}x{K}")
+    g2, beta2 = pkg.ops.fused_g_beta(c[:, N - 2 * Hv:N - Hv].contiguous(), c[:, N - Hv:].contiguous(), A_log, dt_bias,
+                                     None)
+    torch.cuda.synchronize()
+    assert torch.equal(g, g2) and torch.equal(beta.view(torch.int16), beta2.view(torch.int16))
+
+
 @pytest.mark.parametrize("pad,off", [(40, 8), (41, 3)])
 def test_gemm_strided_operands_and_out(pkg, dev, pad, off):
     """Row strides larger than K (views of wider buffers) and an output view;
