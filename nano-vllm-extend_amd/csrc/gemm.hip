@@ -17,6 +17,8 @@
 //   gemm_tn_pp_kernel    256 x 256 tiles, the last few as 128 x 128 quarters;
 //                        8 waves in two alternating groups, persistent (most
 //                        shapes with more than a few hundred rows)
+//   gemm_tn_ring_kernel  16, 32 or 64 rows x 32 columns, K dealt to the waves,
+//                        a load ring per wave (few tiles: a decode out_proj)
 //   gemm_tn_deep_kernel  64 x 128 or 64 x 64, three or four LDS stages (a
 //                        decode in_proj)
 //   gemm_tn_kernel       the general one: 256 x 256 or 192 x 256 where K is an
@@ -495,6 +497,8 @@ __device__ __forceinline__ void half_barrier() {
 // s_waitcnt vmcnt(8) lgkmcnt(0): all but the newest 8 loads have landed and
 // every LDS read has returned
 constexpr int kWaitPP = 8 | (7 << 4);
+// s_waitcnt lgkmcnt(0) alone (vmcnt 63)
+constexpr int kWaitLds = 15 | (7 << 4) | (3 << 14);
 
 // LDS offset of granule c of row r in a half tile of B (see the column order
 // below)
@@ -745,6 +749,129 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_tn_pp_kernel(const uint16_
   __builtin_amdgcn_s_waitcnt(0);
 }
 
+// ---- few tiles (the out projection of a decode batch): a ring per wave ----
+// What bounds it: the loads' latency times the bytes in flight.  Workgroup: BM
+// rows x 32 columns of C; the K-steps of 64 are dealt to its NW waves in turn
+// (wave w: steps w, w + NW, ...), each wave loading its steps into a ring of NS
+// stages of its own in LDS, so the loop has no barrier and up to 144 KiB per CU
+// are in flight.  The waves' partial sums are added through LDS in wave order.
+// (Operands loaded straight to registers instead, 16 rows x 64 bytes per load:
+// 1 x 2048 x 4096 14.8 us, 64 x 12352 x 2048 24-75 us against 11; the address
+// unit pays per row.)  Against the 64 x 64 deep kernel: 1 x 2048 x 4096 16.8 ->
+// 6.2 us, 64 rows 17.1 -> 7.9, 200 rows 17.2 -> 11.7; 256 x 2048 x 2048 10.5 ->
+// 8.1.
+template <int BM, int NW, int NS>
+__global__ __launch_bounds__(64 * NW) void gemm_tn_ring_kernel(const uint16_t* __restrict__ A, int64_t lda,
+                                                              const uint16_t* __restrict__ B, int64_t ldb,
+                                                              GemmOut out, int M, int N, int K, GemmGates gt) {
+  static_assert(NS == 2 || NS == 3, "stages");
+  constexpr int MT = BM / 16, BN = 32;
+  constexpr int kStage = (BM + BN) * 128;   // one wave's stage
+  constexpr int kPer = (BM + BN) / 8;       // 1 KiB blocks of it
+  // s_waitcnt vmcnt: the oldest stage has landed, the loads of the NS - 1 newer
+  // ones stay in flight (lgkmcnt 15: no wait)
+  constexpr int kVm = (NS - 1) * kPer;
+  static_assert(kVm < 64, "vmcnt field");
+  constexpr int kWait = (kVm & 15) | (7 << 4) | (15 << 8) | ((kVm >> 4) << 14);
+  typedef gdn::s16x8_t frag_t;
+  __shared__ __align__(16) uint8_t st0[NW * kStage];
+  __shared__ __align__(16) uint8_t st1[NW * kStage];
+  __shared__ __align__(16) uint8_t st2[NS == 3 ? NW * kStage : 16];
+  __shared__ __align__(16) uint16_t gscr[NW][16 * 32];
+  static_assert(MT * 2048 <= kStage, "the partial sums fit a stage");
+  const int mb_n = (M + BM - 1) / BM, nb_n = (N + BN - 1) / BN;
+  // the row blocks of a column block on one XCD, so that its L2 reads the weights once
+  const int64_t L = gdn::xcd_remap(blockIdx.x, static_cast<int64_t>(mb_n) * nb_n);
+  if (L < 0) return;
+  const int m0 = BM * static_cast<int>(L % mb_n), n0 = BN * static_cast<int>(L / mb_n);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  const __amdgpu_buffer_rsrc_t ra = rsrc_of(A), rb = rsrc_of(B);
+  int goff[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    if (i < BM / 8) {
+      const int gcol = 8 * ((lane & 7) ^ (((i & 1) << 2) | (lane >> 4)));
+      goff[i] = static_cast<int>((min(m0 + 8 * i + (lane >> 3), M - 1) * lda + gcol) * 2);
+    } else {
+      const int b = i - BM / 8;
+      const int gcol = 8 * ((lane & 7) ^ (((b & 3) << 1) | ((lane >> 4) & 1)));
+      goff[i] = static_cast<int>((min(n0 + 8 * b + (lane >> 3), N - 1) * ldb + gcol) * 2);
+    }
+  }
+  const int nk = K / kBK;
+  auto issue = [&](uint8_t* st, int step) {
+    const int kbyte = 128 * min(step, nk - 1);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) dma16(i < BM / 8 ? ra : rb, st + wave * kStage + i * 1024, goff[i], kbyte);
+  };
+  gdn::f32x4_t acc[MT][2];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) acc[i][t] = gdn::f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto one = [&](uint8_t* st, int step) {
+    const uint8_t* a = st + wave * kStage;
+    const uint8_t* b = a + BM * 128;
+    frag_t fa[2][MT], fb[2][2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        fa[ks][i] = *reinterpret_cast<const frag_t*>(a + sw_off(16 * i + lr, 4 * ks + lg));
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        fb[ks][t] = *reinterpret_cast<const frag_t*>(b + swb_off(8 * (lr >> 2) + 4 * t + (lr & 3), 4 * ks + lg));
+    }
+    // the reads have returned before the stage is loaded again
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(kWaitLds);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(st, step + NS * NW);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[i][t] = gdn::mfma16x16x32(fb[ks][t], fa[ks][i], acc[i][t]);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(kWait);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  issue(st0, wave);
+  issue(st1, wave + NW);
+  if constexpr (NS == 3) issue(st2, wave + 2 * NW);
+  __builtin_amdgcn_s_waitcnt(kWait);
+  int s = wave;
+  for (; s + (NS - 1) * NW < nk; s += NS * NW) {
+    one(st0, s);
+    one(st1, s + NW);
+    if constexpr (NS == 3) one(st2, s + 2 * NW);
+  }
+  if (s < nk) one(st0, s);
+  if (NS == 3 && s + NW < nk) one(st1, s + NW);
+  // the repeated loads past the last step land before the stages are reused
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  gdn::f32x4_t* red = reinterpret_cast<gdn::f32x4_t*>(st0);  // [wave][row tile][column tile][lane]
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) red[((wave * MT + i) * 2 + t) * 64 + lane] = acc[i][t];
+  __syncthreads();
+  for (int i = wave; i < MT; i += NW) {
+    gdn::f32x4_t c0 = red[(i * 2) * 64 + lane], c1 = red[(i * 2 + 1) * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) {
+      c0 += red[((w * MT + i) * 2) * 64 + lane];
+      c1 += red[((w * MT + i) * 2 + 1) * 64 + lane];
+    }
+    gemm_store16(c0, c1, out, M, N, m0 + 16 * i, n0, lane, gt, gscr[wave]);
+  }
+}
+
 // ---- small M (decode batches): a deeper load pipeline ----
 // gemm_tn_kernel's two stages let a step's loads arrive during one step's
 // products, which at 64-row tiles are four to eight products: every step then
@@ -928,6 +1055,22 @@ int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, 
   // fewer their prologue and the repeated last loads cost more than they save:
   // 1000 x 2080 x 512: 6.5 -> 7.0 us).
   const bool deep = K / kBK >= 16;
+  // Ring tiles of 16, 32 or 64 rows x 32 columns, the smallest with at most one
+  // workgroup per CU (with more, the 64-row tiles below move fewer bytes: 64 x
+  // 12352 x 2048 11.2 us against 16-19; 500 x 2048 x 2048 13.7 against 13.9).
+  int rows = 16;
+  const int64_t nb32 = (N + 31) / 32;
+  while (rows <= 64 && (M + rows - 1) / rows * nb32 > kCUs) rows *= 2;
+  if (deep && rows <= 64) {
+    const dim3 gr = grid((M + rows - 1) / rows * nb32);
+    if (rows == 16)
+      gemm_tn_ring_kernel<16, 4, 3><<<gr, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+    else if (rows == 32)
+      gemm_tn_ring_kernel<32, 4, 3><<<gr, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+    else
+      gemm_tn_ring_kernel<64, 4, 3><<<gr, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+    return gdn_launch_status();
+  }
   // 64 x 128 tiles, two or more workgroups per CU, spread the work over the
   // whole chip; 64 x 64 when even those would not.
   if (t64x128 >= kCUs / 2) {

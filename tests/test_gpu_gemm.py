@@ -56,11 +56,14 @@ def test_gemm_against_fp32_matmul(pkg, dev, M, N, K):
 # The 8-wave kernel's quarters alone (128 x 128; K of 2, 4 and 6 steps, ragged
 # rows and columns, an empty quarter past M), behind whole tiles, and whole tiles
 # of an uneven last round; its K restriction (192: gemm_tn_kernel at 256 and 192
-# rows).  Hv > 0: the columns go to four parts with gate outputs
+# rows); the ring kernel at 16, 32 and 64 rows with 16, 17 and 33 steps (dealt to
+# four waves: uneven).  Hv > 0: the columns go to four parts with gate outputs
 # (b and a the last 2 Hv columns).
 @pytest.mark.parametrize("M,N,K,Hv", [(1949, 2048, 128, 0), (1100, 4000, 256, 16), (1153, 2072, 384, 4),
                                       (4100, 4008, 384, 4), (4500, 3000, 256, 0), (8190, 2047, 192, 0),
-                                      (17000, 2048, 192, 0)])
+                                      (17000, 2048, 192, 0), (1, 2048, 1024, 0), (16, 2056, 1088, 4),
+                                      (37, 2048, 2112, 16), (100, 2000, 1024, 8), (200, 2056, 1088, 4),
+                                      (250, 1000, 2112, 4)])
 def test_gemm_kernel_edges(pkg, dev, M, N, K, Hv):
     gen = torch.Generator().manual_seed(M + N + K)
     a = torch.randn(M, K, generator=gen).to(BF16)
