@@ -884,6 +884,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_tn_ring_kernel(const uint16_t* _
 // products in the same order and epilogue as gemm_tn_kernel: the results are
 // the same bits.  Steps past the last one repeat its loads into the unused
 // stages (every path issues the same loads), drained before the epilogue.
+// (Graph-replayed, without an exit inside a loop trip: 37 x 12352 x 2048 11.2
+// -> 10.5 us, 128 rows 15.2 -> 14.4, 200 rows 21.9 -> 21.3.)
 template <int BN, int NS>
 __global__ __launch_bounds__(kGemmThreads, 2) void gemm_tn_deep_kernel(const uint16_t* __restrict__ A, int64_t lda,
                                                                     const uint16_t* __restrict__ B, int64_t ldb,
@@ -974,32 +976,28 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_tn_deep_kernel(const uin
   issue(st0, 0);
   issue(st1, 1);
   if constexpr (NS == 4) issue(st2, 2);
-  // Two rounds of the stages per trip.  The compiler's load counting merges
-  // its state at the loop head and then waits there for all but the newest
-  // step's loads before the first reads (vmcnt(kPer)); within a trip the
-  // barrier's own wait covers every read.
-  for (int s = 0; s < nk; s += 2 * NS) {
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int s0 = s + r * NS;
-      if constexpr (NS == 4) {
-        if (s0 >= nk) break;
-        one(st0, st3, s0);
-        if (s0 + 1 >= nk) break;
-        one(st1, st0, s0 + 1);
-        if (s0 + 2 >= nk) break;
-        one(st2, st1, s0 + 2);
-        if (s0 + 3 >= nk) break;
-        one(st3, st2, s0 + 3);
-      } else {
-        if (s0 >= nk) break;
-        one(st0, st2, s0);
-        if (s0 + 1 >= nk) break;
-        one(st1, st0, s0 + 1);
-        if (s0 + 2 >= nk) break;
-        one(st2, st1, s0 + 2);
-      }
+  // (no exit inside a trip: with one, the compiler's load counting merges its
+  // states at the loop head and waits there for loads that are meant to stay
+  // in flight)
+  int s = 0;
+  if constexpr (NS == 4) {
+    for (; s + 3 < nk; s += 4) {
+      one(st0, st3, s);
+      one(st1, st0, s + 1);
+      one(st2, st1, s + 2);
+      one(st3, st2, s + 3);
     }
+    if (s < nk) one(st0, st3, s);
+    if (s + 1 < nk) one(st1, st0, s + 1);
+    if (s + 2 < nk) one(st2, st1, s + 2);
+  } else {
+    for (; s + 2 < nk; s += 3) {
+      one(st0, st2, s);
+      one(st1, st0, s + 1);
+      one(st2, st1, s + 2);
+    }
+    if (s < nk) one(st0, st2, s);
+    if (s + 1 < nk) one(st1, st0, s + 1);
   }
   // the repeated loads land before a stage is reused as the gates' scratch
   __builtin_amdgcn_s_waitcnt(0);
