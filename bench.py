@@ -450,7 +450,7 @@ def decode_bench(pkg, cfg, dev, K, W):
 def decode_gva_bench(pkg, dev, K, W):
     """Config 2's decode step at Qwen3.5's grouped geometry (16 key heads, 32
     value heads; pool [512, 32, 128, 128]), B = 256.  Two heads share each key
-    head, so the step is two launches: the q/k decode conv, then the fused
+    head; at this batch the step is two launches: the q/k decode conv, then the fused
     kernel (gates, v conv with its roll, state update, gated norm).  Returns
     (s per step cold, fused kernel us, tile pass us).  (The q/k conv is not
     burst-timed on its own: at 16 MB a launch it is shorter than a call's
@@ -495,9 +495,9 @@ def recurrent_burst_us(pkg, cfg, core, x, a, b, ids, conv_pool, s_pool, z_rows, 
     sets = [ids, torch.tensor(other, device=ids.device)] if len(other) == B else [ids]
     if core.sw.fused_decode:
         # the kernel the decode step runs: the whole step (q/k/v conv, gates,
-        # state update, norm) with one key head per value head and whole heads
-        # per workgroup, else gates + v conv + state update after the q/k conv
-        whole = Hk == Hv and B * Hv >= pkg.ops.WHOLE_HEAD_TILES
+        # state update, norm) where it runs in one launch, else gates + v conv +
+        # state update after the q/k conv
+        whole = pkg.ops.one_launch_decode(B, Hk, Hv)
         qk = None if whole else pkg.ops.conv_decode_step(x[:, :2 * kd], conv_pool[:, :2 * kd], ids,
                                                            core.conv_w[:2 * kd])
 
@@ -505,7 +505,8 @@ def recurrent_burst_us(pkg, cfg, core, x, a, b, ids, conv_pool, s_pool, z_rows, 
 
         def launch(sl):
             pkg.ops.recurrent_decode_fused(qk, x, conv_pool, core.conv_w, b, a, core.A_log, core.dt_bias, s_pool,
-                                           sl, Hk, Hv, D, z=zz, norm_weight=core.norm_w, eps=core.eps)
+                                           sl, Hk, Hv, D, z=zz, norm_weight=core.norm_w, eps=core.eps,
+                                           grouped=True)
     else:
         g, beta = pkg.ops.fused_g_beta(b, a, core.A_log, core.dt_bias, None)
         y = pkg.ops.conv_decode_step(x, conv_pool, ids, core.conv_w)
@@ -883,8 +884,8 @@ def main():
         extra["decode_gva_16_32_b256"] = {
             "ms_per_step": round(tg * 1e3, 4),
             "what": "config 2's step at Hk = 16, Hv = 32 (Qwen3.5's grouped geometry), B = 256, pool "
-                    "[512, 32, 128, 128], slot sets alternating as in decode_config2: two launches (the q/k decode "
-                    "conv, then the fused kernel)",
+                    "[512, 32, 128, 128], slot sets alternating as in decode_config2 (at this batch two launches: "
+                    "the q/k decode conv, then the fused kernel)",
             "kernels_us": {"recurrent_decode_fused": round(rec_g, 2)},
             "roofline": {"bound": "hbm", "achieved": round(sb_g / (rec_g * 1e-6) / 1e9, 1), "peak": HBM_PEAK_GBPS,
                          "unit": "GB/s", "frac": round(sb_g / (rec_g * 1e-6) / 1e9 / HBM_PEAK_GBPS, 4),

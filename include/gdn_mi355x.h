@@ -293,11 +293,8 @@ int gdn_recurrent(const uint16_t* q, int64_t sq_b, int64_t sq_t, const uint16_t*
  *          the same kernel and o receives its output instead of the core
  *          output, the same bits as gdn_rmsnorm_gated on that core output:
  *          z [B, Hv*D] bf16 gate rows (row stride sz_b), norm_w [D] bf16.
- *          The kernel then runs whole heads per workgroup, as it does without
- *          z from B*Hv >= 2048; below that it otherwise splits a head's
- *          columns over workgroups, which sums S^T k in another order
- * One launch; each v channel (and with q == k == NULL each q and k channel)
- * belongs to one workgroup, which rolls its taps.
+ * One launch; each v channel belongs to one
+ * workgroup, which rolls its taps.  (q == k == NULL: gdn_decode_step.)
  */
 int gdn_recurrent_decode_fused(const uint16_t* q, int64_t sq_b, const uint16_t* k, int64_t sk_b,
                                const uint16_t* x, int64_t sx_row, uint16_t* conv_pool, int64_t cp_slot,
@@ -306,6 +303,22 @@ int gdn_recurrent_decode_fused(const uint16_t* q, int64_t sq_b, const uint16_t* 
                                int64_t s_stride, const int64_t* ids, uint16_t* o, int B, int Hk, int Hv, int D,
                                float scale, int l2norm, const uint16_t* z, int64_t sz_b, const uint16_t* norm_w,
                                float eps, void* stream);
+
+/*
+ * The whole decode step of the layer core in one launch, with one or two value
+ * heads per key head (Hv == Hk or Hv == 2*Hk, else GDN_ERR_UNSUPPORTED): the
+ * decode conv + SiLU of all C channels with their conv-state roll, the gates,
+ * the in-place recurrent update and, with z, the gated RMSNorm
+ * (nanovllm/models/qwen3_5.py:1008-1030, :1083-1085).  The same bits as
+ * gdn_conv_decode over the q and k channels followed by
+ * gdn_recurrent_decode_fused.  The arguments are that entry point's, without
+ * q and k; x is 16-byte aligned with a row stride that is a multiple of 8.
+ */
+int gdn_decode_step(const uint16_t* x, int64_t sx_row, uint16_t* conv_pool, int64_t cp_slot, int64_t cp_ch,
+                    const uint16_t* conv_w, const uint16_t* a, const uint16_t* b, const void* A_log,
+                    const void* dt_bias, int param_is_fp32, float* s_pool, int64_t s_stride, const int64_t* ids,
+                    uint16_t* o, int B, int Hk, int Hv, int D, float scale, int l2norm, const uint16_t* z,
+                    int64_t sz_b, const uint16_t* norm_w, float eps, void* stream);
 
 /*
  * Speculative-verify commit: pool[ids[b]] <- inter[b, accepted[b] - 1]

@@ -57,6 +57,8 @@ SIGNATURES: dict[str, list] = {
     "gdn_recurrent_decode_fused": [_p, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _i32,
                                    _p, _i64, _p, _p, _i32, _i32, _i32, _i32, _f32, _i32, _p, _i64, _p, _f32,
                                    _p],
+    "gdn_decode_step": [_p, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _i32, _p, _i64, _p, _p, _i32, _i32, _i32, _i32,
+                        _f32, _i32, _p, _i64, _p, _f32, _p],
     "gdn_state_commit": [_p, _i64, _p, _p, _p, _i32, _i32, _i32, _i32, _p],
     "gdn_gemm_bf16": [_p, _i64, _p, _i64, _p, _i64, _i32, _i32, _i32, _p, _p, _p, _p, _i32, _i32, _i32, _p],
     "gdn_gemm_bf16_cols": [_p, _i64, _p, _i64, _i32, _i32, _i32, _i32, _p, _p, _p, _p, _p, _p, _p, _i32, _i32,

@@ -35,8 +35,8 @@ With NANOVLLM_GDN_FUSED_DECODE=1 (the default) it replaces
 Qwen3_5GatedDeltaNet._gdn_padded (qwen3_5.py:967-1085) with one whose
 T == 1 branch runs ops.recurrent_decode_fused (gates, the conv with its
 roll, the in-place recurrent update and the gated norm self.norm in one
-kernel, after the q/k decode conv's own launch when the heads are grouped;
-the same results bit for bit); other T keep the original method.
+kernel, after the q/k decode conv's own launch with more than two value heads
+per key head; the same results bit for bit); other T keep the original method.
 
 Both methods read the module's _USE_GDN_GBETA and _USE_CONV_TRITON (and the
 decode method _USE_GDN_INPLACE) on every call, as the reference's layer
@@ -109,16 +109,16 @@ def _fused_decode_method(mod, orig):
         proj = self.in_proj_qkv(x).reshape(-1, self.conv_dim)
         w = self.conv1d.weight.view(self.conv_dim, 4)
         kd = self.key_dim
-        # one key head per value head and whole heads per workgroup: the q/k
-        # conv runs in the decode kernel too; else as its own launch first
+        # one or two value heads per key head: the q/k conv runs in the decode
+        # kernel too; else as its own launch first
         qk = None
-        if not (self.num_k_heads == Hv and n * Hv >= ops.WHOLE_HEAD_TILES):
+        if not ops.one_launch_decode(n, self.num_k_heads, Hv):
             qk = ops.conv_decode_step(proj[:, :2 * kd], self.conv_cache[:, :2 * kd], ids, w[:2 * kd])
         # gates + v conv + in-place update + the gated norm (self.norm's
         # weight and eps) in one kernel
         core = ops.recurrent_decode_fused(qk, proj, self.conv_cache, w, b, a, A_log, dt_bias, self.s_cache, ids,
                                           self.num_k_heads, Hv, self.head_k_dim, z=z.reshape(n, Hv * Dv),
-                                          norm_weight=self.norm.weight, eps=self.norm.eps)
+                                          norm_weight=self.norm.weight, eps=self.norm.eps, grouped=True)
         return self.out_proj(core.reshape(n, 1, self.value_dim))
 
     return _gdn_padded

@@ -578,15 +578,31 @@ def recurrent_gdn_inplace(q, k, v, g, beta, s_pool, ids):
     return _recurrent(q, k, v, g, beta, s_pool, s_pool, ids, None, None, True)
 
 
-# The decode kernel splits each head's columns over NVB workgroups when the
-# batch has few (sequence, head) tiles (NVB 1 from B * Hv >= 2048); the split
-# changes the summation order of S^T k, so whole-head and split runs differ
-# in the last bits.  Its fused norm epilogue needs whole heads.
+# (sequence, head) tiles from which every recurrent kernel runs whole heads per
+# workgroup.  With fewer the head's columns may be split over workgroups: in the
+# multi-token kernel that changes the summation order of S^T k, so its
+# whole-head and split runs differ in the last bits; one-token steps add in one
+# order at every split.
 WHOLE_HEAD_TILES = 2048
 
 
+# With two value heads per key head the one-launch step holds two state tiles per
+# workgroup; from about this many tiles on, the q/k conv's own launch costs no
+# more than the smaller workgroups of the two-launch form gain (32 value heads,
+# graph-replayed core: 32 rows 37.2 us in two launches, 29.6 in one; 64 rows 58.4
+# and 53.7; 150 rows 117.0 and 116.3; 200 rows 149.0 and 149.1; 256 rows 187.2
+# and 189.0).
+GROUPED_STEP_TILES = 5120
+
+
+def one_launch_decode(B: int, num_k_heads: int, num_v_heads: int) -> bool:
+    """Whether the whole decode step, q/k conv included, runs in one kernel:
+    with one value head per key head always, with two at small batches."""
+    return num_v_heads == num_k_heads or (num_v_heads == 2 * num_k_heads and B * num_v_heads < GROUPED_STEP_TILES)
+
+
 def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bias, s_pool, ids, Hk, Hv, D,
-                           scale=None, z=None, norm_weight=None, eps=1e-6, fuse_norm=None):
+                           scale=None, z=None, norm_weight=None, eps=1e-6, fuse_norm=None, grouped=False):
     """The decode step after the q/k conv, in one kernel: the gates from a, b,
     the v channels' conv1d + SiLU (their conv state rolled in place at `ids`)
     and the in-place recurrent update.  qk [B, 2*Hk*D] is conv_decode_step's
@@ -597,14 +613,11 @@ def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bi
     (nanovllm/models/qwen3_5.py:1008-1030).  With z ([B, Hv*D] bf16, head
     dim contiguous) and norm_weight ([D]) `out` is the layer's gated RMSNorm
     of it (qwen3_5.py:1083-1085), the same bits as rms_norm_gated on the core
-    output: in the same kernel when B * Hv >= WHOLE_HEAD_TILES (the kernel
-    runs whole heads then anyway), else as a second launch (fuse_norm=True
-    forces the one-kernel form, whose core output is then the whole-head
-    kernel's).
+    output, in the same kernel (fuse_norm=False: as a second launch).
 
-    qk=None (Hk == Hv only): the q and k channels' decode conv runs in the
-    kernel as well, their conv states rolled there (the whole step in one
-    launch, whole heads per workgroup); the same bits as conv_decode_step on
+    qk=None (Hk == Hv; with grouped also Hv == 2 * Hk): the q and k channels'
+    decode conv runs in the kernel as well, their conv states rolled there
+    (the whole step in one launch); the same bits as conv_decode_step on
     those channels followed by the call above with its output."""
     dev = _check_cuda(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bias, s_pool, ids, z, norm_weight)
     for t, nm in ((qk, "qk"), (mixed, "mixed"), (conv_pool, "conv_pool"), (b, "b"), (a, "a")):
@@ -614,8 +627,9 @@ def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bi
     kd = Hk * D
     assert C == 2 * kd + Hv * D
     if qk is None:
-        assert Hk == Hv, "the q/k conv runs in the decode kernel only with one key head per value head"
-        fuse_norm = True   # whole heads per workgroup in any case
+        assert Hk == Hv or (grouped and Hv == 2 * Hk), \
+            "the q/k conv runs in the decode kernel only with one key head per value head (grouped: per two)"
+        fuse_norm = True
     else:
         assert qk.shape == (B, 2 * kd) and qk.stride(1) == 1
     assert mixed.stride(1) == 1 and conv_pool.stride(2) == 1
@@ -630,7 +644,7 @@ def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bi
     assert _state_view_ok(s_pool, Hv, D)
     ids64 = ids.to(torch.int64).contiguous()
     assert ids64.shape == (B,), "one slot id per row"
-    if z is not None and not (fuse_norm if fuse_norm is not None else B * Hv >= WHOLE_HEAD_TILES):
+    if z is not None and fuse_norm is not None and not fuse_norm:
         core = recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bias, s_pool, ids, Hk, Hv,
                                       D, scale)
         return rms_norm_gated(core, z.reshape(B, 1, Hv, D), norm_weight, eps)
@@ -645,10 +659,13 @@ def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bi
     out = torch.empty(B, 1, Hv, D, dtype=mixed.dtype, device=mixed.device)
     if scale is None:
         scale = D ** -0.5
-    q_ptr, k_ptr, sqk = (None, None, 0) if qk is None else (_lib.ptr(qk), _lib.ptr(qk[:, kd:]), qk.stride(0))
-    _lib.call("gdn_recurrent_decode_fused", q_ptr, sqk, k_ptr, sqk,
-              _lib.ptr(mixed), mixed.stride(0), _lib.ptr(conv_pool), conv_pool.stride(0), conv_pool.stride(1),
-              _lib.ptr(w), _lib.ptr(a), _lib.ptr(b), _lib.ptr(a_log), _lib.ptr(dt_bias),
+    entry, q_k = "gdn_recurrent_decode_fused", (None, 0, None, 0)
+    if qk is not None:
+        q_k = (_lib.ptr(qk), qk.stride(0), _lib.ptr(qk[:, kd:]), qk.stride(0))
+    elif Hk != Hv:
+        entry, q_k = "gdn_decode_step", ()
+    _lib.call(entry, *q_k, _lib.ptr(mixed), mixed.stride(0), _lib.ptr(conv_pool), conv_pool.stride(0),
+              conv_pool.stride(1), _lib.ptr(w), _lib.ptr(a), _lib.ptr(b), _lib.ptr(a_log), _lib.ptr(dt_bias),
               int(a_log.dtype == torch.float32), _lib.ptr(s_pool), s_pool.stride(0), _lib.ptr(ids64),
               _lib.ptr(out), B, Hk, Hv, D, float(scale), 1, _lib.ptr(z), z.stride(0) if z is not None else 0,
               _lib.ptr(nw), float(eps), _stream(dev))

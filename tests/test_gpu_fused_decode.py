@@ -182,3 +182,37 @@ def test_fused_decode_qk_conv_needs_one_key_head_per_value_head(pkg, dev):
         t.to(dev) for t in _case(65, Hk, Hv, D, B, slots, False))
     with pytest.raises(AssertionError):
         pkg.ops.recurrent_decode_fused(None, mixed, conv_pool, conv_w, b, a, A_log, dt_bias, s_pool, ids, Hk, Hv, D)
+
+
+# (D = 64 and 128; one row, an odd batch, and one beyond two workgroups per CU;
+# with and without the norm; the pool a strided per-layer view)
+@pytest.mark.parametrize("Hk,Hv,D,B,norm", [(1, 2, 128, 1, True), (2, 4, 128, 5, False), (16, 32, 128, 37, True),
+                                            (2, 4, 64, 3, True), (4, 8, 64, 150, False), (3, 3, 128, 2, True)],
+                         ids=lambda c: str(c))
+def test_one_launch_decode_step(pkg, dev, Hk, Hv, D, B, norm):
+    """The whole step in one launch with one or two value heads per key head
+    (grouped): bit-equal to fused_g_beta -> conv_decode_step ->
+    recurrent_gdn_inplace -> rms_norm_gated, every channel's taps rolled once,
+    other slots and layers untouched."""
+    ops = pkg.ops
+    slots, layers = B + 3, 2
+    mixed, conv_w, A_log, dt_bias, a, b, conv0, s0, ids = (t.to(dev) for t in _case(67, Hk, Hv, D, B, slots, False))
+    kd = Hk * D
+    gen = torch.Generator().manual_seed(68)
+    z = torch.randn(B, Hv * D, generator=gen).to(BF16).to(dev) if norm else None
+    w = (1 + 0.1 * torch.randn(D, generator=gen)).to(BF16).to(dev) if norm else None
+    cps, sps = conv0[:, None].repeat(1, layers, 1, 1), s0[:, None].repeat(1, layers, 1, 1, 1)
+    cp, sp = cps[:, 1], sps[:, 1]
+    out = ops.recurrent_decode_fused(None, mixed, cp, conv_w, b, a, A_log, dt_bias, sp, ids, Hk, Hv, D, z=z,
+                                     norm_weight=w, grouped=True)
+    g, beta = ops.fused_g_beta(b, a, A_log, dt_bias, None)
+    y = ops.conv_decode_step(mixed, conv0, ids, conv_w)
+    q, k, v = y[:, :kd].view(B, 1, Hk, D), y[:, kd:2 * kd].view(B, 1, Hk, D), y[:, 2 * kd:].view(B, 1, Hv, D)
+    before = s0.clone()
+    ref = ops.recurrent_gdn_inplace(q, k, v, g.view(B, 1, Hv), beta.view(B, 1, Hv), s0, ids)
+    if norm:
+        ref = ops.rms_norm_gated(ref, z.view(B, 1, Hv, D), w, 1e-6)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), "output"
+    assert torch.equal(sp, s0) and torch.equal(cp.view(torch.int16), conv0.view(torch.int16)), "pools"
+    assert torch.equal(sps[:, 0], before), "another layer"
