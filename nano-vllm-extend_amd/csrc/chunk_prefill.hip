@@ -1972,22 +1972,21 @@ __global__ __launch_bounds__(256) void seg_scan_kernel(ScanList sl, int Hv) {
 }
 
 // The scan at D = 128 on the fp32 matrix cores: workgroup (chain, head, 16
-// state columns); wave w computes rows 32 w .. 32 w + 31 of
-// S_{s+1}[:, block] = P_s S_s[:, block] + R_s[:, block] as two 16 x 16 tiles
-// of v_mfma_f32_16x16x4_f32 over the 32 key steps (lane (c, g) holds A
-// element (row c, key 4 kk + g), B element (key 4 kk + g, column c), C rows
-// 4 g + i of column c).  P_s goes through LDS once per step (row pitch D + 4
-// floats: the 64 lanes of an A read hit distinct banks); S_s is re-staged in
-// LDS between steps; P_s and R_s are loaded one step ahead, as in the VALU
-// form above.  (Config 3's scan: 45 us in the VALU form at D = 128.)
-__global__ __launch_bounds__(256) void seg_scan_mfma_kernel(ScanList sl, int Hv) {
+// state columns) of 8 waves; wave w computes rows 16 w .. 16 w + 15 of
+// S_{s+1}[:, block] = P_s S_s[:, block] + R_s[:, block], 32 products of
+// v_mfma_f32_16x16x4_f32.  Product (j, i) takes key 16 j + 4 g + i from lane
+// group g, so that a lane's A elements are eight float4 of one row of P_s: they
+// go straight from L2 (the 8 blocks of a head share one XCD's) to registers, the
+// next step's as soon as this one's are used.  S_s goes round through LDS, two
+// buffers, one barrier per step.  What bounds it: the latency of a step's chain
+// (LDS, 32 dependent products in two accumulators).  Seven steps at 16 heads: 27.4
+// us before (P_s staged through LDS, four waves of 64 products each).
+__global__ __launch_bounds__(512) void seg_scan_mfma_kernel(ScanList sl, int Hv) {
   constexpr int D = 128;
   constexpr int CB = 16;
   constexpr int NB = D / CB;
-  constexpr int PL = D + 4;
-  constexpr int NV = D * D / 4 / 256;  // float4 loads of P per thread
-  __shared__ __align__(16) float Ps[D * PL];
-  __shared__ __align__(16) float Ss[D][CB];
+  constexpr int NJ = D / 16;
+  __shared__ __align__(16) float Ss[2][D][CB + 4];  // (rows 4 g apart on distinct banks)
   const int64_t wi = gdn::xcd_remap(blockIdx.x, static_cast<int64_t>(sl.n) * Hv * NB);
   if (wi < 0) return;
   const int blk = static_cast<int>(wi % NB);
@@ -1999,60 +1998,49 @@ __global__ __launch_bounds__(256) void seg_scan_mfma_kernel(ScanList sl, int Hv)
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int lc = lane & 15, lg = lane >> 4;
-  for (int e = tid; e < D * CB; e += 256) Ss[e / CB][e % CB] = c.S[hp + static_cast<int64_t>(e / CB) * D + blk * CB + e % CB];
-  // the lane's C elements: rows r0 + 16 t + i, column lc
-  const int r0 = 32 * wave + 4 * lg;
+  // the lane's C elements: rows r0 + i, column lc; its A row: 16 w + lc
+  const int r0 = 16 * wave + 4 * lg;
   const int64_t coff = hp + static_cast<int64_t>(r0) * D + blk * CB + lc;
-  // P_s as float4 per thread (row-major: float4 f = tid + 256 i is row f / 32,
-  // columns 4 (f % 32) ..) and the lane's 8 elements of R_s, one step ahead
-  const f32x4_t* pg = reinterpret_cast<const f32x4_t*>(c.P + hp) + tid;
+  const f32x4_t* pg = reinterpret_cast<const f32x4_t*>(c.P + hp + static_cast<int64_t>(16 * wave + lc) * D + 4 * lg);
   const float* rg = c.R + coff;
-  f32x4_t pre[NV];
-  float rpre[8];
+  f32x4_t pre[NJ];
+  float rpre[4];
 #pragma unroll
-  for (int i = 0; i < NV; ++i) pre[i] = pg[256 * i];
+  for (int j = 0; j < NJ; ++j) pre[j] = pg[4 * j];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) rpre[j] = rg[static_cast<int64_t>(16 * (j >> 2) + (j & 3)) * D];
-  gdn::keep_loads_here();
+  for (int i = 0; i < 4; ++i) rpre[i] = rg[static_cast<int64_t>(i) * D];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) Ss[0][r0 + i][lc] = c.S[coff + static_cast<int64_t>(i) * D];
   for (int s = 0; s < c.m; ++s) {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int f = tid + 256 * i;
-      *reinterpret_cast<f32x4_t*>(&Ps[(f >> 5) * PL + 4 * (f & 31)]) = pre[i];
-    }
-    f32x4_t acc0 = {rpre[0], rpre[1], rpre[2], rpre[3]};
-    f32x4_t acc1 = {rpre[4], rpre[5], rpre[6], rpre[7]};
-    gdn::lds_barrier();  // P_s and S_s are in LDS
+    const float (*S)[CB + 4] = Ss[s & 1];
+    f32x4_t acc0 = {rpre[0], rpre[1], rpre[2], rpre[3]}, acc1 = {0.f, 0.f, 0.f, 0.f};
+    gdn::lds_barrier();  // S_s is in LDS, and the other buffer has been read
     const int64_t nx = static_cast<int64_t>(min(s + 1, c.m - 1)) * hs;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) pre[i] = pg[nx / 4 + 256 * i];
+    for (int j = 0; j < NJ; ++j) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) rpre[j] = rg[nx + static_cast<int64_t>(16 * (j >> 2) + (j & 3)) * D];
-    gdn::keep_loads_here();
-    const float* pa = &Ps[(32 * wave + lc) * PL + lg];
-#pragma unroll 8
-    for (int kk = 0; kk < D / 4; ++kk) {
-      const float bv = Ss[4 * kk + lg][lc];
-      acc0 = gdn::mfma16x16x4f32(pa[4 * kk], bv, acc0);
-      acc1 = gdn::mfma16x16x4f32(pa[16 * PL + 4 * kk], bv, acc1);
+      for (int i = 0; i < 4; ++i) {
+        f32x4_t& a = (j & 1) ? acc1 : acc0;
+        a = gdn::mfma16x16x4f32(pre[j][i], S[16 * j + 4 * lg + i][lc], a);
+      }
+      pre[j] = pg[nx / 4 + 4 * j];
     }
-    gdn::lds_barrier();  // every row of S_s and P_s is read
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rpre[i] = rg[nx + static_cast<int64_t>(i) * D];
     float* so = c.S + (s + 1) * hs + coff;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      Ss[r0 + i][lc] = acc0[i];
-      Ss[r0 + 16 + i][lc] = acc1[i];
-      so[static_cast<int64_t>(i) * D] = acc0[i];
-      so[static_cast<int64_t>(16 + i) * D] = acc1[i];
+      const float v = acc0[i] + acc1[i];
+      Ss[(s + 1) & 1][r0 + i][lc] = v;
+      so[static_cast<int64_t>(i) * D] = v;
     }
   }
 }
 
 // Segment plan of one call: how many segments each sequence is cut into.
 // Only when few workgroups would run otherwise (n_seqs * Hv * D / 64 < 128) and
-// the host knows the lengths.  max_segments: 0 = automatic (segments of at
-// least 16 chunks, at most one workgroup per CU in the second pass), 1 =
-// never, k >= 2 = up to k segments per sequence.
+// the host knows the lengths.  max_segments: 0 = automatic (below), 1 = never, k
+// >= 2 = up to k segments per sequence.
 inline bool seg_eligible(int n_seqs, int Hv, int D) { return static_cast<int64_t>(n_seqs) * Hv * (D / kCB) < 128; }
 
 // scratch bytes for the segment states of one call (an upper bound)
@@ -2067,31 +2055,75 @@ struct SegPlan {
   bool any = false;
 };
 
+// Times the automatic plan weighs, in microseconds, fitted to graph-replayed
+// state passes of one sequence: one pass over c chunks takes kOneUs + kChunkUs c
+// (16 value heads: 1,500 tokens 40.5 us, 5,000 118); each of the two passes of
+// segments kPassUs, its launch included, and per chunk up to kBusyUs more as its
+// workgroups fill the CUs (65,536 tokens in 9 segments: 2.15 us per chunk); the
+// scan of m steps kScanUs + kScanStepUs m.
+constexpr double kOneUs = 5.5, kChunkUs = 1.45, kPassUs = 8.0, kBusyUs = 0.7, kScanUs = 4.0, kScanStepUs = 1.2;
+
+// The automatic segment length in chunks (0: no segments), by the estimated time
+// of pass 1, scan and pass 3 over the cuts of the longest sequence into 2 ..
+// kMaxSeg segments; every sequence longer than the length is cut by it.  A pass
+// of more workgroups than CUs takes that many rounds.  Measured, 16 value heads,
+// state passes and scan: 2,000 tokens 49.1 us (one pass 52.1; two segments one
+// after the other, as a fixed least length of 16 chunks gave, 66.5), 3,500 59.5
+// (one pass 84.7, 3 segments 84.0), 5,000 69.9 (118, 4 segments 90.7); 1,500
+// stays one pass, 40.5 against 45.3.
+inline int auto_segment_len(const int64_t* nch, int n, int per_item) {
+  const int64_t longest = *std::max_element(nch, nch + n);
+  double best = 0.97 * (kOneUs + kChunkUs * static_cast<double>(longest));
+  int len = 0;
+  for (int S = 2; S <= std::min<int64_t>(kMaxSeg, longest); ++S) {
+    const int64_t L = (longest + S - 1) / S;
+    int64_t first = 0, second = 0, steps = 0;  // items of pass 1, of pass 3; scan steps
+    for (int r = 0; r < n; ++r) {
+      const int64_t k = std::max<int64_t>(1, (nch[r] + L - 1) / L);
+      first += k == 1 ? 1 : k - 1;
+      second += k - 1;
+      steps = std::max(steps, k - 2);
+    }
+    const auto pass = [&](int64_t items) {
+      const int64_t wgs = items * per_item;
+      const double busy = std::min(1.0, static_cast<double>(wgs) / gdn::kNumCu);
+      return static_cast<double>((wgs + gdn::kNumCu - 1) / gdn::kNumCu) *
+             (kPassUs + (kChunkUs + kBusyUs * busy) * static_cast<double>(L));
+    };
+    const double t = pass(first) + pass(second) +
+                     (steps > 0 ? kScanUs + kScanStepUs * static_cast<double>(steps) : 0.0);
+    if (t < best) {
+      best = t;
+      len = static_cast<int>(L);
+    }
+  }
+  return len;
+}
+
 // (over the sequences selected by select_host, all if NULL)
 inline SegPlan plan_segments(const int64_t* cu_host, const uint8_t* select_host, int n_seqs, int Hv, int D,
                              int max_segments, bool have_scratch) {
   SegPlan pl;
+  if (!cu_host || !have_scratch || max_segments == 1 || n_seqs > kMaxChains * 4) return pl;
+  int64_t nch[kMaxChains * 4];  // chunks of the selected sequences
   int n_sel = 0;
-  for (int r = 0; r < n_seqs; ++r) n_sel += !select_host || select_host[r];
-  if (!cu_host || !have_scratch || max_segments == 1 || !seg_eligible(n_sel, Hv, D) || n_seqs > kMaxChains * 4)
-    return pl;
-  const int per_item = Hv * (D / kCB);
+  for (int r = 0; r < n_seqs; ++r)
+    if (!select_host || select_host[r]) nch[n_sel++] = (cu_host[r + 1] - cu_host[r] + kC - 1) / kC;
+  if (n_sel == 0 || !seg_eligible(n_sel, Hv, D)) return pl;
+  const int len = max_segments >= 2 ? 0 : auto_segment_len(nch, n_sel, Hv * (D / kCB));
+  if (max_segments < 2 && len == 0) return pl;
   int pass1 = 0, pass3 = 0, chains = 0;
   for (int r = 0; r < n_seqs; ++r) {
     pl.nseg[r] = 1;
     pl.len[r] = 1;
     if (select_host && !select_host[r]) continue;
-    const int64_t nch = (cu_host[r + 1] - cu_host[r] + kC - 1) / kC;
-    int S = 1;
-    if (max_segments >= 2) {
-      S = static_cast<int>(std::min<int64_t>(std::min(max_segments, kMaxSeg), nch));
-    } else if (nch >= 32) {
-      S = static_cast<int>(std::min<int64_t>(std::min(kMaxSeg, 256 / (per_item * n_sel) + 1), nch / 16));
-    }
+    const int64_t c = (cu_host[r + 1] - cu_host[r] + kC - 1) / kC;
+    int S = max_segments >= 2 ? static_cast<int>(std::min<int64_t>(std::min(max_segments, kMaxSeg), c))
+                              : static_cast<int>((c + len - 1) / len);
     int L = 1;
     if (S >= 2) {
-      L = static_cast<int>((nch + S - 1) / S);
-      S = static_cast<int>((nch + L - 1) / L);  // no empty last segment
+      L = static_cast<int>((c + S - 1) / S);
+      S = static_cast<int>((c + L - 1) / L);  // no empty last segment
     }
     if (S >= 2 && (chains + (S >= 3) > kMaxChains || pass1 + S - 1 > kMaxSegItems ||
                    pass3 + S - 1 > kMaxSegItems))
@@ -2322,7 +2354,7 @@ int launch_chunk(const uint16_t* q, int64_t sq, const uint16_t* k, int64_t sk, c
     const int64_t swork = static_cast<int64_t>(sc.n) * Hv * (D / 16);
     const int64_t sgrid = gdn::kNumXcd * ((swork + gdn::kNumXcd - 1) / gdn::kNumXcd);
     if constexpr (D == 128)
-      seg_scan_mfma_kernel<<<dim3(static_cast<unsigned>(sgrid)), dim3(256), 0, stream>>>(sc, Hv);
+      seg_scan_mfma_kernel<<<dim3(static_cast<unsigned>(sgrid)), dim3(512), 0, stream>>>(sc, Hv);
     else
       seg_scan_kernel<D><<<dim3(static_cast<unsigned>(sgrid)), dim3(256), 0, stream>>>(sc, Hv);
     st = gdn_launch_status();

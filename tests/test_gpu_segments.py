@@ -96,3 +96,27 @@ def test_segmented_fused_prefill(pkg, dev):
     assert_out(o6, o1, "fused segmented vs one pass")
     assert state_rel(s6, s1) < STATE_REL
     assert torch.equal(c6.view(torch.int16), c1.view(torch.int16)), "conv states"
+
+
+# the automatic plan: one pass (a short sequence), the fewest chunks it cuts, a
+# second sequence cut in two beside one that is not, and every sequence cut
+@pytest.mark.parametrize("lens", [[300], [1900], [4000, 1500, 70], [2600, 2500]], ids=str)
+def test_automatic_segments(pkg, dev, lens):
+    """Slowly decaying states (g of a few hundredths), so that the scan's
+    transitions matter: the automatic plan against one pass and the oracle."""
+    gen = torch.Generator().manual_seed(53)
+    Hk, Hv, D = 2, 4, 128
+    N = sum(lens)
+    q, k, v, g, beta = rule_inputs(gen, N, Hk, Hv, D)
+    g = g * 0.02
+    cu = cu_of(lens)
+    h0 = torch.randn(len(lens), Hv, D, D, generator=gen) * 0.1
+    ro, rS = gdn_ref.chunk_varlen(q, k, v, g, beta.float(), cu, h0)
+    cu_h = torch.tensor(cu, dtype=torch.int64)
+    args = (q.to(dev), k.to(dev), v.to(dev), g.to(dev), beta.to(dev), cu_h.to(dev), h0.to(dev))
+    o_s, S_s = pkg.ops.chunk_gated_delta_rule_varlen(*args, cu_seqlens_cpu=cu_h)
+    o_1, S_1 = pkg.ops.chunk_gated_delta_rule_varlen(*args, cu_seqlens_cpu=cu_h, max_segments=1)
+    assert_out(o_s.cpu(), ro.to(BF16), "automatic segments out")
+    assert_state(S_s.cpu(), rS, "automatic segments final")
+    assert_out(o_s.cpu(), o_1.cpu(), "automatic segments vs one pass")
+    assert state_rel(S_s.cpu(), S_1.cpu()) < STATE_REL
