@@ -130,5 +130,6 @@ def ptr(t) -> int | None:
 
 
 def stream_handle(device) -> int:
-    """hipStream_t of torch's current stream on `device`."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of torch's current stream on `device` (a tensor's device:
+    its index is set)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)

@@ -122,6 +122,16 @@ def late_split(lens_q: list[int], Hv: int):
     return res
 
 
+_NOT_TIMED = contextlib.nullcontext()
+
+
+@contextlib.contextmanager
+def _timing(timer, name: str):
+    timer.start(name)
+    yield
+    timer.stop(name)
+
+
 class GatedDeltaNetCore:
     """GDN layer core for one layer's parameters.
 
@@ -154,14 +164,8 @@ class GatedDeltaNetCore:
             raise NotImplementedError("FLA_RECURRENT=0 selects the reference's pure-torch recurrent "
                                       "port, which is not part of this build")
 
-    @contextlib.contextmanager
     def _timed(self, name: str):
-        if self.timer is None:
-            yield
-            return
-        self.timer.start(name)
-        yield
-        self.timer.stop(name)
+        return _NOT_TIMED if self.timer is None else _timing(self.timer, name)
 
     def _to(self, dev):
         if self.conv_w.device != dev:
@@ -187,15 +191,15 @@ class GatedDeltaNetCore:
             g = g.masked_fill(~mask.unsqueeze(-1), 0.0)
         return g, beta
 
-    def _norm(self, core, z):
+    def _norm(self, core, z, out=None):
         with self._timed("rmsnorm_gated"):
-            return ops.rms_norm_gated(core, z, self.norm_w, self.eps)
+            return ops.rms_norm_gated(core, z, self.norm_w, self.eps, out)
 
     # --------------------------------------------------------------- decode --
-    def decode(self, mixed, z, b, a, ids, conv_cache, s_cache, gb=None):
+    def decode(self, mixed, z, b, a, ids, conv_cache, s_cache, gb=None, out=None):
         """One token per row (the T == 1 branch of _gdn_padded, qwen3_5.py:1008-1030).
         mixed [B, C], z [B, Hv*D], b/a [B, Hv]; pools are per-layer views.
-        Returns core [B, Hv, D] bf16."""
+        Returns core [B, Hv, D] bf16 (in `out` where given)."""
         self._to(mixed.device)
         B = mixed.shape[0]
         Hk, Hv, D = self.Hk, self.Hv, self.D
@@ -207,7 +211,7 @@ class GatedDeltaNetCore:
                 with self._timed("recurrent_decode"):
                     out = ops.recurrent_decode_fused(None, mixed, conv_cache, self.conv_w, b, a, self.A_log,
                                                      self.dt_bias, s_cache, ids, Hk, Hv, D, z=z,
-                                                     norm_weight=self.norm_w, eps=self.eps, grouped=True)
+                                                     norm_weight=self.norm_w, eps=self.eps, grouped=True, out=out)
                 return out.view(B, Hv, D)
             # q/k conv, then gates + v conv + recurrent update + gated norm in
             # one kernel (the same results as the calls below)
@@ -215,7 +219,8 @@ class GatedDeltaNetCore:
                 qk = ops.conv_decode_step(mixed[:, :2 * kd], conv_cache[:, :2 * kd], ids, self.conv_w[:2 * kd])
             with self._timed("recurrent_decode"):
                 out = ops.recurrent_decode_fused(qk, mixed, conv_cache, self.conv_w, b, a, self.A_log, self.dt_bias,
-                                                 s_cache, ids, Hk, Hv, D, z=z, norm_weight=self.norm_w, eps=self.eps)
+                                                 s_cache, ids, Hk, Hv, D, z=z, norm_weight=self.norm_w, eps=self.eps,
+                                                 out=out)
             return out.view(B, Hv, D)
         g, beta = self._g_beta(b.contiguous(), a.contiguous(), None, gb)
         if self.sw.conv_kernel:
@@ -231,19 +236,20 @@ class GatedDeltaNetCore:
         g1, b1 = g.view(B, 1, Hv), beta.view(B, 1, Hv)
         if self.sw.inplace:
             with self._timed("recurrent_decode"):
-                out = ops.recurrent_gdn_inplace(q, k, v, g1, b1, s_cache, ids)
+                core = ops.recurrent_gdn_inplace(q, k, v, g1, b1, s_cache, ids)
         else:
-            out, new_s = ops.recurrent_gated_delta_rule(q, k, v, g1, b1, s_cache[ids])
+            core, new_s = ops.recurrent_gated_delta_rule(q, k, v, g1, b1, s_cache[ids])
             s_cache[ids] = new_s
-        return self._norm(out.view(B, Hv, D), z.view(B, Hv, D))
+        return self._norm(core.view(B, Hv, D), z.view(B, Hv, D), out).view(B, Hv, D)
 
     # ------------------------------------------------------- varlen prefill --
-    def prefill_varlen(self, mixed, z, b, a, lens_q, ids, conv_cache, s_cache, fresh=None, gb=None):
+    def prefill_varlen(self, mixed, z, b, a, lens_q, ids, conv_cache, s_cache, fresh=None, gb=None, out=None):
         """Varlen prefill group (_gdn_prefill_varlen, qwen3_5.py:922-965) with the
         conv and recurrent states read / written in the pools at `ids`.
         mixed [N, C], z [N, Hv*D], b/a [N, Hv].  fresh: optional bool [n],
         sequences that start from zero states (their slots need no zeroing
-        beforehand, model_runner.py:305-322).  Returns core [N, Hv, D] bf16."""
+        beforehand, model_runner.py:305-322).  Returns core [N, Hv, D] bf16 (in
+        `out` where given, except with the split state pass)."""
         self._to(mixed.device)
         N = mixed.shape[0]
         Hk, Hv, D = self.Hk, self.Hv, self.D
@@ -259,7 +265,7 @@ class GatedDeltaNetCore:
                 o = ops.conv_chunk_prefill_varlen(mixed, conv_cache, self.conv_w, b, a, self.A_log, self.dt_bias,
                                                   cu64_gpu, s_cache, ids, Hk, Hv, D, fresh=fresh,
                                                   cu_seqlens_cpu=cu64_cpu)
-            return self._norm(o, z.view(N, Hv, D))
+            return self._norm(o, z.view(N, Hv, D), out).view(N, Hv, D)
         if fresh is not None:
             zero = ids[fresh.to(device=ids.device, dtype=torch.bool)]
             conv_cache[zero] = 0
@@ -276,7 +282,7 @@ class GatedDeltaNetCore:
             o, _ = ops.chunk_gated_delta_rule_varlen(q.view(N, Hk, D), k.view(N, Hk, D), v.view(N, Hv, D),
                                                      g, beta, cu64_gpu, s_cache, state_ids=ids,
                                                      final_state=s_cache, cu_seqlens_cpu=cu64_cpu)
-        return self._norm(o, z.view(N, Hv, D))
+        return self._norm(o, z.view(N, Hv, D), out).view(N, Hv, D)
 
     def _prefill_split(self, mixed, z, b, a, lens_q, ids, conv_cache, s_cache, fresh, cu64_cpu, cu64_gpu, split):
         """Fused prefill with the state pass split over two streams: the longest
@@ -405,23 +411,26 @@ class GatedDeltaNetCore:
             n1 += 1
         pre_ok = 0 < n1 < bs and min(lens_q[n1:]) > 1
         if n1 == 0 or pre_ok:
-            parts = []
-            off = 0
+            off = n1
+            # a step with both parts: they write the rows of one output
+            out = torch.empty(N, self.value_dim, dtype=torch.bfloat16, device=mixed.device) if n1 else None
             if n1:
-                parts.append(self.decode(mixed[:n1], z[:n1], b[:n1], a[:n1], ids[:n1], conv_cache,
-                                         s_cache, gb=rows(0, n1)).view(n1, self.value_dim))
-                off = n1
+                self.decode(mixed[:n1], z[:n1], b[:n1], a[:n1], ids[:n1], conv_cache, s_cache, gb=rows(0, n1),
+                            out=out[:n1])
+            rest = None if out is None else out[off:]
             if self.sw.varlen:
-                parts.append(self.prefill_varlen(mixed[off:], z[off:], b[off:], a[off:], lens_q[off:],
-                                                 ids[off:], conv_cache, s_cache,
-                                                 gb=rows(off, N)).view(-1, self.value_dim))
+                core = self.prefill_varlen(mixed[off:], z[off:], b[off:], a[off:], lens_q[off:], ids[off:],
+                                           conv_cache, s_cache, gb=rows(off, N), out=rest).view(-1, self.value_dim)
             else:
                 lens_p = lens_dev()[off:]
                 Tp = T if off == 0 else max(lens_q[off:])
-                parts.append(self._padded_varlen(mixed[off:], z[off:], b[off:], a[off:], lens_p, Tp, ids[off:],
-                                                 conv_cache, s_cache, gb=rows(off, N)))
-            # (one part: no concatenation, which would copy the whole output)
-            return parts[0] if len(parts) == 1 else torch.cat(parts, dim=0)
+                core = self._padded_varlen(mixed[off:], z[off:], b[off:], a[off:], lens_p, Tp, ids[off:],
+                                           conv_cache, s_cache, gb=rows(off, N))
+            if out is None:
+                return core
+            if core.data_ptr() != rest.data_ptr():
+                rest.copy_(core)
+            return out
         # len-1 rows that are not a contiguous prefix: one padded pass
         return self._padded_varlen(mixed, z, b, a, lens_dev(), T, ids, conv_cache, s_cache, gb=gb)
 
@@ -479,17 +488,7 @@ class GatedDeltaNetLayer:
         return self.w_in.shape[0]
 
     def _timed(self, name):
-        t = self.timer
-        if t is None:
-            return contextlib.nullcontext()
-
-        @contextlib.contextmanager
-        def cm():
-            t.start(name)
-            yield
-            t.stop(name)
-
-        return cm()
+        return _NOT_TIMED if self.timer is None else _timing(self.timer, name)
 
     def gates_in_gemm(self) -> bool:
         """Whether a path of the core would run the gate kernel on in_proj's b

@@ -36,6 +36,14 @@ def _bf16(t: torch.Tensor, name: str) -> None:
         raise TypeError(f"{name} must be bfloat16, got {t.dtype}")
 
 
+def _out(t: torch.Tensor, numel: int, dev: torch.device) -> torch.Tensor:
+    """A caller's output tensor, checked."""
+    _bf16(t, "out")
+    if t.device != dev or t.numel() != numel or not t.is_contiguous() or t.data_ptr() % 16:
+        raise ValueError("out must be a contiguous, 16-byte aligned tensor of the result's size on its device")
+    return t
+
+
 def _stream(dev: torch.device) -> int:
     return _lib.stream_handle(dev)
 
@@ -221,6 +229,10 @@ def _host_offsets(cu_cpu, n: int):
     """int64 host copy of the sequence offsets [n + 1], or None."""
     if cu_cpu is None:
         return None
+    if (isinstance(cu_cpu, torch.Tensor) and cu_cpu.dtype == torch.int64
+            and cu_cpu.device.type == "cpu" and cu_cpu.is_contiguous()):
+        assert cu_cpu.shape == (n + 1,)
+        return cu_cpu
     t = torch.as_tensor(cu_cpu)
     if t.device.type != "cpu":
         raise ValueError("cu_seqlens_cpu must be in host memory")
@@ -602,7 +614,8 @@ def one_launch_decode(B: int, num_k_heads: int, num_v_heads: int) -> bool:
 
 
 def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bias, s_pool, ids, Hk, Hv, D,
-                           scale=None, z=None, norm_weight=None, eps=1e-6, fuse_norm=None, grouped=False):
+                           scale=None, z=None, norm_weight=None, eps=1e-6, fuse_norm=None, grouped=False,
+                           out=None):
     """The decode step after the q/k conv, in one kernel: the gates from a, b,
     the v channels' conv1d + SiLU (their conv state rolled in place at `ids`)
     and the in-place recurrent update.  qk [B, 2*Hk*D] is conv_decode_step's
@@ -618,7 +631,8 @@ def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bi
     qk=None (Hk == Hv; with grouped also Hv == 2 * Hk): the q and k channels'
     decode conv runs in the kernel as well, their conv states rolled there
     (the whole step in one launch); the same bits as conv_decode_step on
-    those channels followed by the call above with its output."""
+    those channels followed by the call above with its output.  out: a
+    contiguous bf16 tensor of B * Hv * D elements that takes the result."""
     dev = _check_cuda(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bias, s_pool, ids, z, norm_weight)
     for t, nm in ((qk, "qk"), (mixed, "mixed"), (conv_pool, "conv_pool"), (b, "b"), (a, "a")):
         if t is not None:
@@ -647,7 +661,7 @@ def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bi
     if z is not None and fuse_norm is not None and not fuse_norm:
         core = recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bias, s_pool, ids, Hk, Hv,
                                       D, scale)
-        return rms_norm_gated(core, z.reshape(B, 1, Hv, D), norm_weight, eps)
+        return rms_norm_gated(core, z.reshape(B, 1, Hv, D), norm_weight, eps, out)
     nw = None
     if z is not None:
         _bf16(z, "z")
@@ -656,7 +670,10 @@ def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bi
             z = z.contiguous()
         assert norm_weight is not None and norm_weight.numel() == D
         nw = norm_weight.to(torch.bfloat16).contiguous()
-    out = torch.empty(B, 1, Hv, D, dtype=mixed.dtype, device=mixed.device)
+    if out is None:
+        out = torch.empty(B, 1, Hv, D, dtype=mixed.dtype, device=mixed.device)
+    else:
+        out = _out(out, B * Hv * D, dev).view(B, 1, Hv, D)
     if scale is None:
         scale = D ** -0.5
     entry, q_k = "gdn_recurrent_decode_fused", (None, 0, None, 0)
@@ -907,10 +924,11 @@ def linear_cols(x: torch.Tensor, weight: torch.Tensor, widths: list[int],
 
 # -------------------------------------------------------------- gated norm --
 def rms_norm_gated(hidden_states: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor,
-                   eps: float) -> torch.Tensor:
+                   eps: float, out: torch.Tensor | None = None) -> torch.Tensor:
     """y = bf16(float(bf16(w * bf16(x * rsqrt(mean(x^2) + eps)))) * silu(float(z)))
     over the last dim.  hidden_states / gate [..., H, D] bf16 (head dim
-    contiguous, rows of a token contiguous).
+    contiguous, rows of a token contiguous).  out: a contiguous bf16 tensor of as
+    many elements that takes the result.
     Reference: _rms_gated_forward, nanovllm/models/qwen3_5.py:121-131."""
     dev = _check_cuda(hidden_states, gate, weight)
     _bf16(hidden_states, "hidden_states")
@@ -927,7 +945,10 @@ def rms_norm_gated(hidden_states: torch.Tensor, gate: torch.Tensor, weight: torc
     if z2.stride(2) != 1 or z2.stride(1) != D:
         z2 = z2.contiguous()
     n_tok, H, _ = x2.shape
-    y = torch.empty(n_tok, H, D, dtype=hidden_states.dtype, device=hidden_states.device)
+    if out is None:
+        y = torch.empty(n_tok, H, D, dtype=hidden_states.dtype, device=hidden_states.device)
+    else:
+        y = _out(out, n_tok * H * D, dev)
     _lib.call("gdn_rmsnorm_gated", _lib.ptr(x2), x2.stride(0), _lib.ptr(z2), z2.stride(0), _lib.ptr(w),
               _lib.ptr(y), n_tok, H, D, float(eps), _stream(dev))
     return y.view(hidden_states.shape)
