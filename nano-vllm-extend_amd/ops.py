@@ -679,7 +679,8 @@ def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bi
     entry, q_k = "gdn_recurrent_decode_fused", (None, 0, None, 0)
     if qk is not None:
         q_k = (_lib.ptr(qk), qk.stride(0), _lib.ptr(qk[:, kd:]), qk.stride(0))
-    elif Hk != Hv:
+    elif grouped and (Hk != Hv or B * Hv < WHOLE_HEAD_TILES):
+        # (takes the rows that the q/k conv's own launch takes, and no others)
         entry, q_k = "gdn_decode_step", ()
     _lib.call(entry, *q_k, _lib.ptr(mixed), mixed.stride(0), _lib.ptr(conv_pool), conv_pool.stride(0),
               conv_pool.stride(1), _lib.ptr(w), _lib.ptr(a), _lib.ptr(b), _lib.ptr(a_log), _lib.ptr(dt_bias),
