@@ -120,3 +120,23 @@ def test_automatic_segments(pkg, dev, lens):
     assert_state(S_s.cpu(), rS, "automatic segments final")
     assert_out(o_s.cpu(), o_1.cpu(), "automatic segments vs one pass")
     assert state_rel(S_s.cpu(), S_1.cpu()) < STATE_REL
+
+
+# empty sequences at the start, between others and at the end; lengths around a
+# chunk; the most sequences that the host's list holds, and one more
+@pytest.mark.parametrize("D,lens", [(128, [0, 1, 64, 0, 0, 65, 130, 3, 63, 128, 5, 200, 0]),
+                                    (64, [70, 0, 1, 129] * 5), (128, [17, 0, 66, 64] * 16), (128, [17, 0, 66, 64] * 16 + [9])],
+                         ids=lambda c: str(len(c)) if isinstance(c, list) else str(c))
+def test_listed_chunks(pkg, dev, D, lens):
+    """Chunks located from the host's list: the same bits as from the device's
+    offsets alone."""
+    gen = torch.Generator().manual_seed(54)
+    Hk = Hv = 16
+    q, k, v, g, beta = rule_inputs(gen, sum(lens), Hk, Hv, D)
+    cu = torch.tensor(cu_of(lens), dtype=torch.int64)
+    h0 = torch.randn(len(lens), Hv, D, D, generator=gen) * 0.1
+    args = (q.to(dev), k.to(dev), v.to(dev), g.to(dev), beta.to(dev), cu.to(dev), h0.to(dev))
+    o_h, S_h = pkg.ops.chunk_gated_delta_rule_varlen(*args, cu_seqlens_cpu=cu)
+    o_d, S_d = pkg.ops.chunk_gated_delta_rule_varlen(*args)
+    assert torch.equal(o_h.view(torch.int16), o_d.view(torch.int16)), "outputs"
+    assert torch.equal(S_h, S_d), "states"
