@@ -216,3 +216,19 @@ def test_one_launch_decode_step(pkg, dev, Hk, Hv, D, B, norm):
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), "output"
     assert torch.equal(sp, s0) and torch.equal(cp.view(torch.int16), conv0.view(torch.int16)), "pools"
     assert torch.equal(sps[:, 0], before), "another layer"
+
+
+@pytest.mark.parametrize("Hk,Hv", [(2, 2), (2, 4)])
+def test_one_launch_decode_step_row_alignment(pkg, dev, Hk, Hv):
+    """Rows that are not 16 bytes apart are refused before any launch, as the
+    q/k conv's own launch refuses them."""
+    D, B = 64, 3
+    mixed, conv_w, A_log, dt_bias, a, b, conv_pool, s_pool, ids = (
+        t.to(dev) for t in _case(69, Hk, Hv, D, B, B + 1, False))
+    C = mixed.shape[1]
+    rows = torch.zeros(B, C + 4, dtype=BF16, device=dev)[:, :C]
+    with pytest.raises(pkg._lib.GDNKernelError):
+        pkg.ops.conv_decode_step(rows[:, :2 * Hk * D], conv_pool[:, :2 * Hk * D], ids, conv_w[:2 * Hk * D])
+    with pytest.raises(pkg._lib.GDNKernelError):
+        pkg.ops.recurrent_decode_fused(None, rows, conv_pool, conv_w, b, a, A_log, dt_bias, s_pool, ids, Hk, Hv, D,
+                                       grouped=True)
