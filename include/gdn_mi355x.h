@@ -187,10 +187,13 @@ int gdn_set_column_split(int mode);
  *   phase  3 = the whole call; 1 = the prep kernel only; 2 = the state pass
  *          only (after a phase-1 call with the same arguments and workspace,
  *          ordered after it on the caller's side: the two state calls of a
- *          split may run on different streams)
+ *          split may run on different streams, each sequence's segment states
+ *          having their own part of the workspace)
  *   select_host  uint8 [n_seqs] in host memory or NULL: the state pass runs
  *          only the selected sequences (needs cu_seqlens_host, n_seqs <= 64);
- *          each sequence's state pass, conv roll included, must run exactly once
+ *          each sequence's state pass, conv roll included, must run exactly once.
+ *          The segments are planned over all sequences, so the results are the
+ *          whole call's, bit for bit
  * Two launches, as gdn_chunk_prefill: the prep kernel also runs the gates and
  * the q and k channels' conv of its chunk; the state kernel runs the v
  * channels' conv and rolls the conv states.

@@ -2071,10 +2071,13 @@ __global__ __launch_bounds__(512) void seg_scan_mfma_kernel(ScanList sl, int Hv)
 // >= 2 = up to k segments per sequence.
 inline bool seg_eligible(int n_seqs, int Hv, int D) { return static_cast<int64_t>(n_seqs) * Hv * (D / kCB) < 128; }
 
-// scratch bytes for the segment states of one call (an upper bound)
+// scratch bytes for the segment states of one call: a slice of kSegStates states
+// for each sequence (S, P and R of kMaxSeg segments), so that launches over
+// disjoint selections of a call's sequences may run at the same time
+constexpr int kSegStates = 3 * kMaxSeg - 5;
 inline int64_t seg_scratch_bytes(int n_seqs, int Hv, int D) {
   if (!seg_eligible(n_seqs, Hv, D)) return 0;
-  return static_cast<int64_t>(n_seqs) * (3 * kMaxSeg - 5) * Hv * D * D * 4;
+  return static_cast<int64_t>(n_seqs) * kSegStates * Hv * D * D * 4;
 }
 
 struct SegPlan {
@@ -2128,24 +2131,22 @@ inline int auto_segment_len(const int64_t* nch, int n, int per_item) {
   return len;
 }
 
-// (over the sequences selected by select_host, all if NULL)
-inline SegPlan plan_segments(const int64_t* cu_host, const uint8_t* select_host, int n_seqs, int Hv, int D,
-                             int max_segments, bool have_scratch) {
+// (over all sequences of the call, whichever a launch selects: the selections of
+// a split state pass then cut each sequence as one launch would, and give its
+// bits)
+inline SegPlan plan_segments(const int64_t* cu_host, int n_seqs, int Hv, int D, int max_segments, bool have_scratch) {
   SegPlan pl;
-  if (!cu_host || !have_scratch || max_segments == 1 || n_seqs > kMaxChains * 4) return pl;
-  int64_t nch[kMaxChains * 4];  // chunks of the selected sequences
-  int n_sel = 0;
-  for (int r = 0; r < n_seqs; ++r)
-    if (!select_host || select_host[r]) nch[n_sel++] = (cu_host[r + 1] - cu_host[r] + kC - 1) / kC;
-  if (n_sel == 0 || !seg_eligible(n_sel, Hv, D)) return pl;
-  const int len = max_segments >= 2 ? 0 : auto_segment_len(nch, n_sel, Hv * (D / kCB));
+  if (!cu_host || !have_scratch || max_segments == 1 || n_seqs > kMaxChains * 4 || !seg_eligible(n_seqs, Hv, D))
+    return pl;
+  int64_t nch[kMaxChains * 4];  // the sequences' chunks
+  for (int r = 0; r < n_seqs; ++r) nch[r] = (cu_host[r + 1] - cu_host[r] + kC - 1) / kC;
+  const int len = max_segments >= 2 ? 0 : auto_segment_len(nch, n_seqs, Hv * (D / kCB));
   if (max_segments < 2 && len == 0) return pl;
   int pass1 = 0, pass3 = 0, chains = 0;
   for (int r = 0; r < n_seqs; ++r) {
     pl.nseg[r] = 1;
     pl.len[r] = 1;
-    if (select_host && !select_host[r]) continue;
-    const int64_t c = (cu_host[r + 1] - cu_host[r] + kC - 1) / kC;
+    const int64_t c = nch[r];
     int S = max_segments >= 2 ? static_cast<int>(std::min<int64_t>(std::min(max_segments, kMaxSeg), c))
                               : static_cast<int>((c + len - 1) / len);
     int L = 1;
@@ -2281,7 +2282,7 @@ int launch_chunk(const uint16_t* q, int64_t sq, const uint16_t* k, int64_t sk, c
     first[r] = static_cast<int>(total);
     total += (cu_host[r + 1] - cu_host[r] + kC - 1) / kC;
   }
-  const SegPlan pl = plan_segments(cu_host, select_host, n_seqs, Hv, D, max_segments, seg_ws != nullptr);
+  const SegPlan pl = plan_segments(cu_host, n_seqs, Hv, D, max_segments, seg_ws != nullptr);
   SegList plan;
   if (!pl.any && !select_host) plan = plan_columns(cu_host, first, n_seqs, Hv, D);
   // (without a plan all offsets come from the device)
@@ -2361,9 +2362,8 @@ int launch_chunk(const uint16_t* q, int64_t sq, const uint16_t* k, int64_t sk, c
     none.n = 0;
     return state_launch(none, n_seqs);
   }
-  // segment states: per split sequence S_1 .. S_{m+1}, P_1 .. P_m, R_1 .. R_m
+  // segment states: in each split sequence's slice S_1 .. S_{m+1}, P_1 .. P_m, R_1 .. R_m
   const int64_t hs = static_cast<int64_t>(Hv) * D * D;
-  float* scratch = reinterpret_cast<float*>(seg_ws);
   SegList p1, p3;
   p1.n = 0;
   p3.n = 0;
@@ -2379,10 +2379,9 @@ int launch_chunk(const uint16_t* q, int64_t sq, const uint16_t* k, int64_t sk, c
       continue;
     }
     const int m = S - 2;
-    float* Sst = scratch;  // S_1 .. S_{m+1}
+    float* Sst = reinterpret_cast<float*>(seg_ws) + static_cast<int64_t>(r) * kSegStates * hs;
     float* P = Sst + (m + 1) * hs;
     float* R = P + m * hs;
-    scratch = R + m * hs;
     p1.it[p1.n++] = item(r, 0, L, kSegOut, 1, 0, nullptr, Sst);
     for (int s = 1; s <= m; ++s)
       p1.it[p1.n++] = item(r, s * L, (s + 1) * L, kSegBoth, 0, 0, nullptr, R + (s - 1) * hs, P + (s - 1) * hs);

@@ -140,3 +140,36 @@ def test_listed_chunks(pkg, dev, D, lens):
     o_d, S_d = pkg.ops.chunk_gated_delta_rule_varlen(*args)
     assert torch.equal(o_h.view(torch.int16), o_d.view(torch.int16)), "outputs"
     assert torch.equal(S_h, S_d), "states"
+
+
+# both selections cut into several segments; one of a very long sequence; D = 64
+@pytest.mark.parametrize("Hk,Hv,D,lens,late", [(2, 4, 128, [2600, 2300, 70], [True, False, False]),
+                                               (2, 2, 64, [70, 3300, 0, 2500], [False, True, False, False]),
+                                               (16, 16, 128, [49675, 1893, 573], [True, False, False])], ids=str)
+def test_split_state_pass_segments(pkg, dev, Hk, Hv, D, lens, late):
+    """The state pass of a segmented call split over two launches, whose segment
+    states have their own places: the same launches in order on one stream, and
+    the whole call, give the same bits (slowly decaying states, so that every
+    segment state matters)."""
+    gen = torch.Generator(device=dev).manual_seed(55)
+    N, n = sum(lens), len(lens)
+    C = 2 * Hk * D + Hv * D
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device=dev)
+    mixed, conv_w = rand(N, C).to(BF16), (rand(C, 4) * 0.5).to(BF16)
+    a, b = rand(N, Hv).to(BF16), rand(N, Hv).to(BF16)
+    A_log, dt_bias = (rand(Hv) * 0.3 - 4).to(BF16), rand(Hv).to(BF16)
+    conv0, s0 = rand(n + 1, C, 3).to(BF16), rand(n + 1, Hv, D, D) * 0.1
+    ids = torch.randperm(n + 1, generator=gen, device=dev)[:n]
+    cu = torch.tensor(cu_of(lens), dtype=torch.int64)
+    outs = []
+    for side in (None, torch.cuda.current_stream(dev), torch.cuda.Stream(dev)):
+        cp, sp, keep = conv0.clone(), s0.clone(), []
+        res = pkg.ops.conv_chunk_prefill_varlen(mixed, cp, conv_w, b, a, A_log, dt_bias, cu.to(dev), sp, ids, Hk, Hv,
+                                                D, cu_seqlens_cpu=cu, late=None if side is None else late,
+                                                side_stream=side, keep=keep)
+        torch.cuda.synchronize()
+        outs.append((res if side is None else res[0], cp, sp))
+    for name, (o, cp, sp) in zip(("in order", "two streams"), outs[1:]):
+        assert torch.equal(o.view(torch.int16), outs[0][0].view(torch.int16)), f"{name}: outputs"
+        assert torch.equal(cp.view(torch.int16), outs[0][1].view(torch.int16)), f"{name}: conv states"
+        assert torch.equal(sp, outs[0][2]), f"{name}: states"
