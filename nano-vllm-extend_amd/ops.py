@@ -662,12 +662,15 @@ def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bi
         core = recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bias, s_pool, ids, Hk, Hv,
                                       D, scale)
         return rms_norm_gated(core, z.reshape(B, 1, Hv, D), norm_weight, eps, out)
-    nw = None
+    nw, sz = None, 0
     if z is not None:
         _bf16(z, "z")
         z = z.reshape(B, Hv * D)
-        if z.stride(1) != 1 or z.stride(0) % 4:
+        # (rows that overlap, as of one gate row expanded over the batch, are
+        # copied too: the kernel takes whole rows)
+        if z.stride(1) != 1 or (B > 1 and (z.stride(0) % 4 or z.stride(0) < Hv * D)):
             z = z.contiguous()
+        sz = z.stride(0) if B > 1 else Hv * D
         assert norm_weight is not None and norm_weight.numel() == D
         nw = norm_weight.to(torch.bfloat16).contiguous()
     if out is None:
@@ -685,8 +688,7 @@ def recurrent_decode_fused(qk, mixed, conv_pool, conv_weight, b, a, a_log, dt_bi
     _lib.call(entry, *q_k, _lib.ptr(mixed), mixed.stride(0), _lib.ptr(conv_pool), conv_pool.stride(0),
               conv_pool.stride(1), _lib.ptr(w), _lib.ptr(a), _lib.ptr(b), _lib.ptr(a_log), _lib.ptr(dt_bias),
               int(a_log.dtype == torch.float32), _lib.ptr(s_pool), s_pool.stride(0), _lib.ptr(ids64),
-              _lib.ptr(out), B, Hk, Hv, D, float(scale), 1, _lib.ptr(z), z.stride(0) if z is not None else 0,
-              _lib.ptr(nw), float(eps), _stream(dev))
+              _lib.ptr(out), B, Hk, Hv, D, float(scale), 1, _lib.ptr(z), sz, _lib.ptr(nw), float(eps), _stream(dev))
     return out
 
 

@@ -232,3 +232,23 @@ def test_one_launch_decode_step_row_alignment(pkg, dev, Hk, Hv):
     with pytest.raises(pkg._lib.GDNKernelError):
         pkg.ops.recurrent_decode_fused(None, rows, conv_pool, conv_w, b, a, A_log, dt_bias, s_pool, ids, Hk, Hv, D,
                                        grouped=True)
+
+
+@pytest.mark.parametrize("B", [1, 3])
+@pytest.mark.parametrize("Hk,Hv,one", [(2, 4, False), (2, 4, True), (2, 8, False), (4, 4, True)])
+def test_fused_decode_norm_expanded_gate(pkg, dev, Hk, Hv, one, B):
+    """One gate row for every decode row (row stride 0), as the norm's own launch
+    takes it: the same bits as with the rows written out."""
+    ops, D = pkg.ops, 64
+    mixed, conv_w, A_log, dt_bias, a, b, conv0, s0, ids = (t.to(dev) for t in _case(70, Hk, Hv, D, B, B + 2, False))
+    gen = torch.Generator().manual_seed(71)
+    z = torch.randn(Hv * D, generator=gen).to(BF16).to(dev).expand(B + 1, Hv * D)[:B]
+    w = (1 + 0.1 * torch.randn(D, generator=gen)).to(BF16).to(dev)
+    kd = Hk * D
+    outs = []
+    for zz in (z, z.clone(memory_format=torch.contiguous_format)):
+        cp, sp = conv0.clone(), s0.clone()
+        qk = None if one else ops.conv_decode_step(mixed[:, :2 * kd], cp[:, :2 * kd], ids, conv_w[:2 * kd])
+        outs.append(ops.recurrent_decode_fused(qk, mixed, cp, conv_w, b, a, A_log, dt_bias, sp, ids, Hk, Hv, D, z=zz,
+                                               norm_weight=w, grouped=True))
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
