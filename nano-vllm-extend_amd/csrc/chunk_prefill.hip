@@ -2087,24 +2087,24 @@ struct SegPlan {
 };
 
 // Times the automatic plan weighs, in microseconds, fitted to graph-replayed
-// state passes of one sequence: one pass over c chunks takes kOneUs + kChunkUs c
-// (16 value heads: 1,500 tokens 40.5 us, 5,000 118); each of the two passes of
-// segments kPassUs, its launch included, and per chunk up to kBusyUs more as its
-// workgroups fill the CUs (65,536 tokens in 9 segments: 2.15 us per chunk); the
-// scan of m steps kScanUs + kScanStepUs m.
-constexpr double kOneUs = 5.5, kChunkUs = 1.45, kPassUs = 8.0, kBusyUs = 0.7, kScanUs = 4.0, kScanStepUs = 1.2;
+// calls of 12 to 400 chunks cut into 1 to 12 segments each: 4 to 32 value heads,
+// one to three sequences, D = 64 and 128 (which differ by less than the fit).
+// One pass over c chunks takes kOneUs + kChunkUs c; each of the two passes of
+// segments kPassUs, its launch included, and kSegUs per chunk, up to kBusyUs more
+// as its workgroups fill the CUs; the scan of m steps kScanUs + kScanStepUs m.
+constexpr double kOneUs = 5.5, kChunkUs = 1.45, kPassUs = 5.0, kSegUs = 1.7, kBusyUs = 0.8, kScanUs = 3.0,
+                 kScanStepUs = 3.0;
 
 // The automatic segment length in chunks (0: no segments), by the estimated time
 // of pass 1, scan and pass 3 over the cuts of the longest sequence into 2 ..
 // kMaxSeg segments; every sequence longer than the length is cut by it.  A pass
-// of more workgroups than CUs takes that many rounds.  Measured, 16 value heads,
-// state passes and scan: 2,000 tokens 49.1 us (one pass 52.1; two segments one
-// after the other, as a fixed least length of 16 chunks gave, 66.5), 3,500 59.5
-// (one pass 84.7, 3 segments 84.0), 5,000 69.9 (118, 4 segments 90.7); 1,500
-// stays one pass, 40.5 against 45.3.
+// of more workgroups than CUs takes that many rounds.  Measured, whole calls at
+// 16 value heads: 26 chunks stay one pass, 64.3 us (cut, 68 to 78); 30 70.0 in one
+// pass and 68.4 in the plan's six segments, 48 98.0 and 83.6, 128 224 and 138; 24
+// and 18 chunks at 8 heads stay one pass, 60.4 (cut, 62 to 85).
 inline int auto_segment_len(const int64_t* nch, int n, int per_item) {
   const int64_t longest = *std::max_element(nch, nch + n);
-  double best = 0.97 * (kOneUs + kChunkUs * static_cast<double>(longest));
+  double best = kOneUs + kChunkUs * static_cast<double>(longest);
   int len = 0;
   for (int S = 2; S <= std::min<int64_t>(kMaxSeg, longest); ++S) {
     const int64_t L = (longest + S - 1) / S;
@@ -2119,7 +2119,7 @@ inline int auto_segment_len(const int64_t* nch, int n, int per_item) {
       const int64_t wgs = items * per_item;
       const double busy = std::min(1.0, static_cast<double>(wgs) / gdn::kNumCu);
       return static_cast<double>((wgs + gdn::kNumCu - 1) / gdn::kNumCu) *
-             (kPassUs + (kChunkUs + kBusyUs * busy) * static_cast<double>(L));
+             (kPassUs + (kSegUs + kBusyUs * busy) * static_cast<double>(L));
     };
     const double t = pass(first) + pass(second) +
                      (steps > 0 ? kScanUs + kScanStepUs * static_cast<double>(steps) : 0.0);

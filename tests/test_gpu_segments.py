@@ -122,6 +122,24 @@ def test_automatic_segments(pkg, dev, lens):
     assert state_rel(S_s.cpu(), S_1.cpu()) < STATE_REL
 
 
+# lengths that one pass runs faster than any cut: 26 chunks at 16 heads, 24 and 18
+# at 8; lengths that segments run faster: 32 and 48 chunks
+@pytest.mark.parametrize("Hk,Hv,D,lens,cut", [(16, 16, 128, [1661], False), (16, 32, 64, [1661], False),
+                                              (4, 8, 128, [1533, 1132], False), (16, 16, 128, [2045], True),
+                                              (16, 16, 64, [3070], True)], ids=str)
+def test_automatic_plan_lengths(pkg, dev, Hk, Hv, D, lens, cut):
+    """Whether the automatic plan cuts: its bits are the one-pass call's or not
+    (slowly decaying states, whose roundings differ between the two)."""
+    gen = torch.Generator().manual_seed(56)
+    q, k, v, g, beta = rule_inputs(gen, sum(lens), Hk, Hv, D, slow_decay=True)
+    cu = torch.tensor(cu_of(lens), dtype=torch.int64)
+    h0 = torch.randn(len(lens), Hv, D, D, generator=gen) * 0.1
+    args = (q.to(dev), k.to(dev), v.to(dev), g.to(dev), beta.to(dev), cu.to(dev), h0.to(dev))
+    S_a = pkg.ops.chunk_gated_delta_rule_varlen(*args, cu_seqlens_cpu=cu)[1]
+    S_1 = pkg.ops.chunk_gated_delta_rule_varlen(*args, cu_seqlens_cpu=cu, max_segments=1)[1]
+    assert torch.equal(S_a, S_1) != cut
+
+
 # empty sequences at the start, between others and at the end; lengths around a
 # chunk; the most sequences that the host's list holds, and one more
 @pytest.mark.parametrize("D,lens", [(128, [0, 1, 64, 0, 0, 65, 130, 3, 63, 128, 5, 200, 0]),
