@@ -86,6 +86,16 @@ def test_gemm_kernel_edges(pkg, dev, M, N, K, Hv):
     assert torch.equal(g, g2) and torch.equal(beta.view(torch.int16), beta2.view(torch.int16))
 
 
+# The 8-wave kernel without whole tiles, over the 128 x 128 blocks of C: 3 x 65
+# blocks with ragged edges, 16 x 16, 9 x 28 and 10 x 17 (a partial last group of
+# rows), 1 x 256 with K of 2 steps; K of 14, 20 and 22 steps (a last round of four
+# steps that ends after two).  Hv > 0: four parts with gate outputs.
+@pytest.mark.parametrize("M,N,K,Hv", [(300, 8224, 1280, 16), (1949, 2048, 896, 0), (1100, 3500, 896, 4),
+                                      (1153, 2072, 1408, 4), (100, 32700, 128, 0)])
+def test_gemm_blocks(pkg, dev, M, N, K, Hv):
+    test_gemm_kernel_edges(pkg, dev, M, N, K, Hv)
+
+
 @pytest.mark.parametrize("pad,off", [(40, 8), (41, 3)])
 def test_gemm_strided_operands_and_out(pkg, dev, pad, off):
     """Row strides larger than K (views of wider buffers) and an output view;
