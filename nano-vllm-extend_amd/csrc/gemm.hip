@@ -1036,13 +1036,25 @@ int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, 
     return dim3(static_cast<unsigned>(gdn::kNumXcd * ((wgs + gdn::kNumXcd - 1) / gdn::kNumXcd)));
   };
   const dim3 b3(kGemmThreads);
-  // 256 x 256 tiles when they fill half of the CUs, or quarters of them when
-  // those make one round that fills more than half (1949 x 2048 x 4096: 42.6
-  // -> 37.7 us against 64 x 128 tiles, 900 x 4096 x 2048 23.9 -> 22.4, 256 x
-  // 8224 x 2048 20.1 -> 19.8; two rounds of quarters do not pay, 400 x 12352 x
-  // 2048: 35.0 -> 38.1).  The two-stage loop takes K in pairs of steps.
+  // The 8-wave kernel (K in pairs of steps) when its 256 x 256 tiles fill half of
+  // the CUs, except where 192 x 256 tiles run in one round as well and there are
+  // few of them, or as few as the 256-row ones, or K is short: the round is then
+  // its rows' time, and the persistent kernel's start is not made up for (900 x
+  // 8224 x 2048: 43.6 us against 41.5 with 192 rows, 257 x 32768 52.0 / 45.6, 3000
+  // x 3000 45.5 / 42.1; 1200 x 8224 44.1 / 45.2; 1200 x 8224 x 512 16.9 / 16.1).
   const bool wide = t256 >= kCUs / 2;
-  if (K % (2 * kBK) == 0 && (wide || (t128 > kCUs / 2 && t128 <= kCUs))) {
+  const bool one192 = t256 > kCUs / 2 && t192 <= kCUs &&
+                      (5 * t192 <= 4 * kCUs || t192 == t256 || K < 16 * kBK);
+  // Fewer tiles: as 128 x 128 blocks in one round.  Against 64 x 128 tiles, two of
+  // them per CU, they take as long for a few blocks as for 256, so these must have
+  // work for more than one tile per CU, few blocks that are half empty, and a K
+  // that makes up for the start (1949 x 2048 x 4096: 42.6 -> 37.7 us, 900 x 4096 x
+  // 2048 23.9 -> 22.4, 384 x 8224 x 2048 22.2 -> 22.0; the other way 129 x 8224 x
+  // 2048 14.4 -> 19.5, 257 x 6144 15.6 -> 20.6, 768 x 4096 x 1024 11.9 -> 12.7, 900 x
+  // 4096 x 512 7.7 -> 9.7; two rounds of blocks, 400 x 12352 x 2048 35.0 -> 38.1).
+  const bool blocks = !wide && t128 <= kCUs && t64x128 > kCUs && 2 * t64x128 > 3 * t128 &&
+                      K * t64x128 >= 1600 * kCUs;
+  if (K % (2 * kBK) == 0 && (wide ? !one192 : blocks)) {
     const int64_t rem = t256 % kCUs;
     const int64_t whole = rem <= kCUs / 2 ? t256 - rem : t256;
     const int64_t wgs = std::min<int64_t>(kCUs, whole ? std::max(whole, 4 * (t256 - whole)) : t128);
@@ -1051,10 +1063,10 @@ int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, 
     return gdn_launch_status();
   }
   if (wide) {
-    // Odd multiples of 64: a launch runs in ceil(tiles / CUs) waves of tiles,
-    // each taking time in proportion to the tile's rows; 192 x 256 is taken when
-    // its waves x rows is smaller (a short last wave of 256-row tiles, e.g. 536
-    // tiles = 2.09 waves -> 712 = 2.78).
+    // Odd multiples of 64, and one round of 192-row tiles: a launch runs in
+    // ceil(tiles / CUs) waves of tiles, each taking time in proportion to the
+    // tile's rows; 192 x 256 is taken when its waves x rows is smaller (a short
+    // last wave of 256-row tiles, e.g. 536 tiles = 2.09 waves -> 712 = 2.78).
     const int64_t w256 = (t256 + kCUs - 1) / kCUs, w192 = (t192 + kCUs - 1) / kCUs;
     if (w192 * 192 < w256 * 256)
       gemm_tn_kernel<192, 256, 1><<<grid(t192), b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);

@@ -96,6 +96,17 @@ def test_gemm_blocks(pkg, dev, M, N, K, Hv):
     test_gemm_kernel_edges(pkg, dev, M, N, K, Hv)
 
 
+# Either side of the 8-wave kernel's lines: 132 tiles of 256 rows and 165 of 192
+# (one round of 192 rows) at K of 2, 14 and 16 steps; 165 and 231 at 14 and 16
+# steps; 260 tiles of 64 x 128 against 130 blocks at 24 and 26 steps, 195 against
+# 130 (half empty blocks).  Whole tiles with a tail of quarters at K of 2 steps.
+@pytest.mark.parametrize("M,N,K,Hv", [(900, 8224, 128, 16), (900, 8224, 896, 0), (900, 8224, 1024, 16),
+                                      (1200, 8224, 896, 0), (1200, 8224, 1024, 4), (256, 8224, 1536, 16),
+                                      (256, 8224, 1664, 16), (129, 8224, 1664, 0), (4100, 4008, 128, 4)])
+def test_gemm_kernel_choice(pkg, dev, M, N, K, Hv):
+    test_gemm_kernel_edges(pkg, dev, M, N, K, Hv)
+
+
 @pytest.mark.parametrize("pad,off", [(40, 8), (41, 3)])
 def test_gemm_strided_operands_and_out(pkg, dev, pad, off):
     """Row strides larger than K (views of wider buffers) and an output view;
