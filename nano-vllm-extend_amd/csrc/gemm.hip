@@ -1080,11 +1080,16 @@ int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, 
   const bool deep = K / kBK >= 16;
   // Ring tiles of 16, 32 or 64 rows x 32 columns, the smallest with at most one
   // workgroup per CU (with more, the 64-row tiles below move fewer bytes: 64 x
-  // 12352 x 2048 11.2 us against 16-19; 500 x 2048 x 2048 13.7 against 13.9).
+  // 12352 x 2048 11.2 us against 16-19; 500 x 2048 x 2048 13.7 against 13.9), and
+  // not 64 rows of an A that is tall and more than the 4 MiB of an XCD's L2: every
+  // XCD reads all of A for its column blocks (2000 x 256 x 2048 13.5 us against
+  // 9.9 with 64 x 64 tiles, 6000 x 64 x 2048 11.4 / 9.6; 1024 x 512 x 2048 9.2 /
+  // 9.9, 1700 x 256 x 1024 6.2 / 6.6; one column block, 16384 x 32 x 1024, 6.3 / 9.0).
   int rows = 16;
   const int64_t nb32 = (N + 31) / 32;
   while (rows <= 64 && (M + rows - 1) / rows * nb32 > kCUs) rows *= 2;
-  if (deep && rows <= 64) {
+  const bool tall = M > 1024 && N > 32 && static_cast<int64_t>(M) * K > (1 << 21);
+  if (deep && rows <= (tall ? 32 : 64)) {
     const dim3 gr = grid((M + rows - 1) / rows * nb32);
     if (rows == 16)
       gemm_tn_ring_kernel<16, 4, 3><<<gr, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);

@@ -100,9 +100,12 @@ def test_gemm_blocks(pkg, dev, M, N, K, Hv):
 # (one round of 192 rows) at K of 2, 14 and 16 steps; 165 and 231 at 14 and 16
 # steps; 260 tiles of 64 x 128 against 130 blocks at 24 and 26 steps, 195 against
 # 130 (half empty blocks).  Whole tiles with a tail of quarters at K of 2 steps.
+# The ring's 64-row tiles: 1024 rows, 4 MiB of A and more, one column block.
 @pytest.mark.parametrize("M,N,K,Hv", [(900, 8224, 128, 16), (900, 8224, 896, 0), (900, 8224, 1024, 16),
                                       (1200, 8224, 896, 0), (1200, 8224, 1024, 4), (256, 8224, 1536, 16),
-                                      (256, 8224, 1664, 16), (129, 8224, 1664, 0), (4100, 4008, 128, 4)])
+                                      (256, 8224, 1664, 16), (129, 8224, 1664, 0), (4100, 4008, 128, 4),
+                                      (1024, 500, 1088, 4), (1500, 200, 1344, 4), (1500, 200, 1408, 0),
+                                      (9000, 24, 1024, 0)])
 def test_gemm_kernel_choice(pkg, dev, M, N, K, Hv):
     test_gemm_kernel_edges(pkg, dev, M, N, K, Hv)
 
