@@ -764,8 +764,8 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_tn_pp_kernel(const uint16_
 
 // ---- few tiles (the out projection of a decode batch): a ring per wave ----
 // What bounds it: the loads' latency times the bytes in flight.  Workgroup: BM
-// rows x 32 columns of C; the K-steps of 64 are dealt to its NW waves in turn
-// (wave w: steps w, w + NW, ...), each wave loading its steps into a ring of NS
+// rows x 32 columns of C; the K-steps of 64 are dealt to its four waves in turn
+// (wave w: steps w, w + 4, ...), each wave loading its steps into a ring of three
 // stages of its own in LDS, so the loop has no barrier and up to 144 KiB per CU
 // are in flight.  The waves' partial sums are added through LDS in wave order.
 // (Operands loaded straight to registers instead, 16 rows x 64 bytes per load:
@@ -773,11 +773,11 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_tn_pp_kernel(const uint16_
 // unit pays per row.)  Against the 64 x 64 deep kernel: 1 x 2048 x 4096 16.8 ->
 // 6.2 us, 64 rows 17.1 -> 7.9, 200 rows 17.2 -> 11.7; 256 x 2048 x 2048 10.5 ->
 // 8.1.
-template <int BM, int NW, int NS>
-__global__ __launch_bounds__(64 * NW) void gemm_tn_ring_kernel(const uint16_t* __restrict__ A, int64_t lda,
-                                                              const uint16_t* __restrict__ B, int64_t ldb,
-                                                              GemmOut out, int M, int N, int K, GemmGates gt) {
-  static_assert(NS == 2 || NS == 3, "stages");
+template <int BM>
+__global__ __launch_bounds__(kGemmThreads) void gemm_tn_ring_kernel(const uint16_t* __restrict__ A, int64_t lda,
+                                                                    const uint16_t* __restrict__ B, int64_t ldb,
+                                                                    GemmOut out, int M, int N, int K, GemmGates gt) {
+  constexpr int NW = kGemmThreads / 64, NS = 3;
   constexpr int MT = BM / 16, BN = 32;
   constexpr int kStage = (BM + BN) * 128;   // one wave's stage
   constexpr int kPer = (BM + BN) / 8;       // 1 KiB blocks of it
@@ -789,7 +789,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_tn_ring_kernel(const uint16_t* _
   typedef gdn::s16x8_t frag_t;
   __shared__ __align__(16) uint8_t st0[NW * kStage];
   __shared__ __align__(16) uint8_t st1[NW * kStage];
-  __shared__ __align__(16) uint8_t st2[NS == 3 ? NW * kStage : 16];
+  __shared__ __align__(16) uint8_t st2[NW * kStage];
   __shared__ __align__(16) uint16_t gscr[NW][16 * 32];
   static_assert(MT * 2048 <= kStage, "the partial sums fit a stage");
   const int mb_n = (M + BM - 1) / BM, nb_n = (N + BN - 1) / BN;
@@ -855,16 +855,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_tn_ring_kernel(const uint16_t* _
   };
   issue(st0, wave);
   issue(st1, wave + NW);
-  if constexpr (NS == 3) issue(st2, wave + 2 * NW);
+  issue(st2, wave + 2 * NW);
   __builtin_amdgcn_s_waitcnt(kWait);
   int s = wave;
   for (; s + (NS - 1) * NW < nk; s += NS * NW) {
     one(st0, s);
     one(st1, s + NW);
-    if constexpr (NS == 3) one(st2, s + 2 * NW);
+    one(st2, s + 2 * NW);
   }
   if (s < nk) one(st0, s);
-  if (NS == 3 && s + NW < nk) one(st1, s + NW);
+  if (s + NW < nk) one(st1, s + NW);
   // the repeated loads past the last step land before the stages are reused
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
@@ -1092,11 +1092,11 @@ int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, 
   if (deep && rows <= (tall ? 32 : 64)) {
     const dim3 gr = grid((M + rows - 1) / rows * nb32);
     if (rows == 16)
-      gemm_tn_ring_kernel<16, 4, 3><<<gr, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+      gemm_tn_ring_kernel<16><<<gr, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
     else if (rows == 32)
-      gemm_tn_ring_kernel<32, 4, 3><<<gr, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+      gemm_tn_ring_kernel<32><<<gr, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
     else
-      gemm_tn_ring_kernel<64, 4, 3><<<gr, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
+      gemm_tn_ring_kernel<64><<<gr, b3, 0, st>>>(A, lda, B, ldb, out, M, N, K, gt);
     return gdn_launch_status();
   }
   // 64 x 128 tiles, two or more workgroups per CU, spread the work over the
