@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define GDN_ABI_VERSION 4
+#define GDN_ABI_VERSION 5
 
 #define GDN_OK 0
 #define GDN_ERR_INVALID_ARG (-1) /* shape / stride / pointer rejected */
@@ -37,7 +37,7 @@ extern "C" {
  * (one per GPU, held until the process ends). */
 #define GDN_NOALLOC_SCRATCH_BYTES (128LL << 20)
 
-/* ABI version of the loaded library (GDN_ABI_VERSION). */
+/* ABI version of the loaded library (GDN_ABI_VERSION; 5 added gdn_decode_step). */
 int gdn_abi_version(void);
 
 /*

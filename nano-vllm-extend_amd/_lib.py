@@ -14,7 +14,7 @@ from pathlib import Path
 import torch  # noqa: F401  (loads the HIP runtime the library binds to)
 
 LIB_PATH = Path(os.environ.get("GDN_MI355X_LIB", Path(__file__).resolve().parent / "lib" / "libgdn_mi355x.so"))
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 GDN_OK = 0
 GDN_ERR_INVALID_ARG = -1

@@ -43,6 +43,20 @@ def test_library_exports_every_declared_symbol(pkg):
     assert lib.gdn_abi_version() == pkg._lib.ABI_VERSION
 
 
+def test_library_without_an_entry_point_is_refused_by_its_version(pkg, monkeypatch, tmp_path):
+    """A library of version 4, from before gdn_decode_step, is refused with the
+    version in the error and not at the missing symbol."""
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    names = set(pkg._lib.SIGNATURES) - {"gdn_abi_version", "gdn_decode_step"}
+    src.write_text("int gdn_abi_version(void) { return 4; }\n"
+                   + "".join(f"int {n}(void) {{ return -1; }}\n" for n in sorted(names)))
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    monkeypatch.setattr(pkg._lib, "LIB_PATH", so)
+    monkeypatch.setattr(pkg._lib, "_LIB", None)
+    with pytest.raises(pkg._lib.GDNLibraryError, match="ABI mismatch: library 4"):
+        pkg._lib.load()
+
+
 def test_bindings_match_header(pkg):
     d = _declared()
     assert set(pkg._lib.SIGNATURES) == set(d)
