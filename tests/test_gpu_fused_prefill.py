@@ -101,6 +101,54 @@ def test_fused_against_oracle(pkg, dev):
     assert torch.equal(cp.cpu()[ids].view(torch.int16), new_conv.view(torch.int16)), "conv pool"
 
 
+@pytest.mark.parametrize("host", [False, True])
+@pytest.mark.parametrize("D", [128, 64])
+def test_two_heads_per_prep_workgroup(pkg, dev, D, host):
+    """32 value heads over 16 key heads with more than 1024 (chunk, value head)
+    pieces, where a prep workgroup runs a key head's two value heads in turn: the
+    chunk rule alone and the fused call against the oracle, and bit for bit
+    against each sequence in a call of its own, small enough for one value head per
+    workgroup; with and without the offsets on the host."""
+    Hk, Hv = 16, 32
+    lens = [0, 1, 65, 700, 130, 64, 900, 640, 0, 63]
+    n, N = len(lens), sum(lens)
+    assert ((N + 63) // 64 + n) * Hv > 1024 and (max(lens) // 64 + 2) * Hv <= 1024
+    C, mixed, conv_w, A_log, dt_bias, a, b, conv_pool, s_pool, ids = _case(44, Hk, Hv, D, lens, n + 2)
+    g, beta = gdn_ref.g_beta(b, a, A_log, dt_bias, None)
+    y, new_conv = gdn_ref.conv_varlen(mixed, conv_pool[ids], conv_w, lens)
+    kd = Hk * D
+    q, k, v = y[:, :kd].reshape(N, Hk, D), y[:, kd:2 * kd].reshape(N, Hk, D), y[:, 2 * kd:].reshape(N, Hv, D)
+    ro, rs = gdn_ref.chunk_varlen(q, k, v, g, beta.float(), cu_of(lens), s_pool[ids])
+    rule = [t.to(dev) for t in (q, k, v, g, beta)]
+    mixed, conv_w, A_log, dt_bias, a, b, idd = (t.to(dev) for t in (mixed, conv_w, A_log, dt_bias, a, b, ids))
+
+    def run(fused, rows, sel, sub, cp, sp):
+        cu = torch.tensor(cu_of(sub), dtype=torch.int64)
+        kw = dict(cu_seqlens_cpu=cu if host else None, max_segments=1)
+        if fused:
+            return pkg.ops.conv_chunk_prefill_varlen(mixed[rows], cp, conv_w, b[rows], a[rows], A_log, dt_bias,
+                                                     cu.to(dev), sp, idd[sel], Hk, Hv, D, **kw)
+        return pkg.ops.chunk_gated_delta_rule_varlen(*(t[rows] for t in rule), cu.to(dev), sp, state_ids=idd[sel],
+                                                     final_state=sp, **kw)[0]
+
+    for fused in (False, True):
+        cp, sp, cp1, sp1 = conv_pool.to(dev), s_pool.to(dev), conv_pool.to(dev), s_pool.to(dev)
+        o = run(fused, slice(0, N), slice(0, n), lens, cp, sp)
+        assert_out(o.cpu(), ro.to(BF16), f"fused {fused} output")
+        assert_state(sp.cpu()[ids], rs, f"fused {fused} state")
+        at = 0
+        for r, t in enumerate(lens):
+            if t:
+                o1 = run(fused, slice(at, at + t), slice(r, r + 1), [t], cp1, sp1)
+                assert torch.equal(o[at:at + t].view(torch.int16), o1.view(torch.int16)), f"sequence {r}: output"
+            at += t
+        assert torch.equal(sp, sp1), "state pool differs"
+        if fused:
+            assert torch.equal(cp.cpu()[ids].view(torch.int16), new_conv.view(torch.int16)), "conv pool vs oracle"
+            written = [int(ids[r]) for r, t in enumerate(lens) if t]
+            assert torch.equal(cp[written].view(torch.int16), cp1[written].view(torch.int16)), "conv pool differs"
+
+
 @pytest.mark.parametrize("Hk,Hv,D,lens", [(4, 4, 128, [1, 2, 70, 3, 0, 129]), (2, 4, 64, [66, 2, 130])],
                          ids=lambda c: str(c))
 def test_fresh_flags_equal_zeroed_slots(pkg, dev, Hk, Hv, D, lens):
