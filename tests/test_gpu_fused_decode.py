@@ -87,9 +87,8 @@ def test_fused_decode_against_oracle(pkg, dev):
 def test_fused_decode_norm_equals_separate_norm(pkg, dev, Hk, Hv, D, B, slots):
     """With the gate rows and the norm weight the decode step also applies the
     layer's gated RMSNorm (qwen3_5.py:1083-1085): bit-equal to
-    recurrent_decode_fused followed by rms_norm_gated, states and conv pool
-    as without the norm.  From B * Hv >= 2048 the norm runs in the decode
-    kernel itself (the last two cases), below it as a second launch."""
+    recurrent_decode_fused followed by rms_norm_gated (also as fuse_norm=False
+    runs it), states and conv pool as without the norm."""
     ops = pkg.ops
     mixed, conv_w, A_log, dt_bias, a, b, conv_pool, s_pool, ids = (
         t.to(dev) for t in _case(63, Hk, Hv, D, B, slots, False))
@@ -112,12 +111,18 @@ def test_fused_decode_norm_equals_separate_norm(pkg, dev, Hk, Hv, D, B, slots):
     assert torch.equal(y2.view(B, Hv, D).view(torch.int16), y1.view(torch.int16)), "fused norm differs"
     assert torch.equal(sp2, sp1), "state pool differs"
     assert torch.equal(cp2.view(torch.int16), cp1.view(torch.int16)), "conv pool differs"
+    cp3, sp3 = conv_pool.clone(), s_pool.clone()
+    qk3 = ops.conv_decode_step(mixed[:, :2 * kd], cp3[:, :2 * kd], ids, conv_w[:2 * kd])
+    y3 = ops.recurrent_decode_fused(qk3, mixed, cp3, conv_w, b, a, A_log, dt_bias, sp3, ids, Hk, Hv, D,
+                                    z=z, norm_weight=w, eps=1e-6, fuse_norm=False)
+    assert torch.equal(y3.view(B, Hv, D).view(torch.int16), y1.view(torch.int16)), "norm as a second launch differs"
+    assert torch.equal(sp3, sp1), "state pool differs"
 
 
 def test_fused_decode_norm_epilogue_small_batch_vs_oracle(pkg, dev):
-    """The in-kernel norm forced at a small batch (whole heads per workgroup
-    where the plain kernel would split them): against the oracle's decode
-    chain and gated norm."""
+    """The in-kernel norm at a small batch (whole heads per workgroup where the
+    kernel without it splits them): against the oracle's decode chain and gated
+    norm."""
     Hk, Hv, D, B, slots = 2, 4, 128, 5, 8
     mixed, conv_w, A_log, dt_bias, a, b, conv_pool, s_pool, ids = _case(65, Hk, Hv, D, B, slots, False)
     gen = torch.Generator().manual_seed(66)
@@ -140,18 +145,17 @@ def test_fused_decode_norm_epilogue_small_batch_vs_oracle(pkg, dev):
     assert torch.equal(cp.cpu().view(torch.int16), rpool.view(torch.int16)), "conv pool"
 
 
-# (B * Hv below the whole-head threshold only with the norm: the reference
-# call then runs whole heads too, as the qk=None kernel always does)
 @pytest.mark.parametrize("Hk,Hv,D,B,slots,with_norm",
                          [(16, 16, 128, 130, 140, False), (16, 16, 128, 130, 140, True),
-                          (8, 8, 64, 260, 270, False), (8, 8, 64, 260, 270, True), (4, 4, 128, 3, 6, True)],
+                          (8, 8, 64, 260, 270, False), (8, 8, 64, 260, 270, True), (4, 4, 128, 3, 6, True),
+                          (4, 4, 128, 3, 6, False), (4, 4, 64, 40, 50, False)],
                          ids=lambda c: str(c))
 def test_fused_decode_with_qk_conv(pkg, dev, Hk, Hv, D, B, slots, with_norm):
     """qk=None: the q/k channels' decode conv and roll run in the decode kernel
     too (one launch for the whole step).  Bit-equal to conv_decode_step on the
-    q/k channels followed by the fused call with its output, in the whole-head
-    form the kernel then runs; conv pools equal over all channels, other
-    slots untouched."""
+    q/k channels followed by the fused call with its output, also where that
+    call splits a head's columns over workgroups; conv pools equal over all
+    channels, other slots untouched."""
     ops = pkg.ops
     mixed, conv_w, A_log, dt_bias, a, b, conv_pool, s_pool, ids = (
         t.to(dev) for t in _case(63, Hk, Hv, D, B, slots, False))

@@ -112,11 +112,11 @@ def _draw_decode(i):
 @pytest.mark.parametrize("i", list(range(16)))
 def test_random_shape_decode(pkg, dev, i):
     """Decode steps of random shapes: the fused step against fused_g_beta ->
-    conv_decode_step -> recurrent_gdn_inplace (-> the gated norm) bit for bit;
-    with one key head per value head also the one-launch form that runs the
-    q/k conv too (bit for bit where both run whole heads per workgroup, else
-    against the two-launch whole-head form); each against the CPU oracle's
-    decode chain (nanovllm/models/qwen3_5.py:1008-1030, :1083-1085)."""
+    conv_decode_step -> recurrent_gdn_inplace (-> the gated norm) bit for bit,
+    the norm in the decode kernel and as its own launch; with one or two value
+    heads per key head also the one-launch form that runs the q/k conv too; the
+    separate calls and the one launch against the CPU oracle's decode chain
+    (nanovllm/models/qwen3_5.py:1008-1030, :1083-1085)."""
     from test_gpu_fused_decode import _case as _dcase
     c = _draw_decode(i)
     Hk, Hv, D, B, slots = c["Hk"], c["Hv"], c["D"], c["B"], c["slots"]
@@ -137,7 +137,6 @@ def test_random_shape_decode(pkg, dev, i):
     if z is not None:
         o1 = ops.rms_norm_gated(o1, z.view(B, Hv, D), w, 1e-6)
     kw = dict(z=z, norm_weight=w, eps=1e-6) if z is not None else {}
-    whole = B * Hv >= ops.WHOLE_HEAD_TILES  # the separate calls' kernel runs whole heads per workgroup
 
     def step(one, **extra):
         cp2, sp2 = conv_pool.clone(), s_pool.clone()
@@ -153,15 +152,13 @@ def test_random_shape_decode(pkg, dev, i):
                                r.view(torch.int16) if r.dtype == BF16 else r), f"{name}: {what}"
 
     same(step(False), (o1, sp1, cp1), "q/k conv first")
-    one = step(True) if Hk == Hv else None
-    if one is not None and whole:
+    if z is not None:
+        same(step(False, fuse_norm=False), (o1, sp1, cp1), "q/k conv first, norm last")
+    one = step(True, grouped=True) if Hv in (Hk, 2 * Hk) else None
+    if one is not None:
         same(one, (o1, sp1, cp1), "one launch")
-    elif one is not None and z is not None:
-        # (with fewer rows the separate calls split a head's columns over
-        # workgroups, whose sums over the rows group differently: the same
-        # results within the bars, other bits; the two-launch form with the
-        # norm in its kernel runs whole heads, as the one launch does)
-        same(one, step(False, fuse_norm=True), "one launch vs two launches with whole heads")
+    if Hk == Hv:
+        same(step(True), (o1, sp1, cp1), "one launch, not grouped")
     # the oracle's decode chain
     mixed_h, conv_w_h, A_log_h, dt_bias_h, a_h, b_h, conv_pool_h, s_pool_h, ids_h = host
     rg, rbeta = gdn_ref.g_beta(b_h, a_h, A_log_h, dt_bias_h, None)
