@@ -140,6 +140,42 @@ def test_automatic_plan_lengths(pkg, dev, Hk, Hv, D, lens, cut):
     assert torch.equal(S_a, S_1) != cut
 
 
+# (float64 on the GPU: 16 or 8 heads, one long sequence or two)
+@pytest.mark.parametrize("Hk,Hv,D,lens", [(16, 16, 128, [2000]), (4, 8, 128, [3500]), (16, 16, 64, [2500, 1900]),
+                                          (16, 16, 128, [5000])], ids=str)
+@pytest.mark.parametrize("decay", [0.02, 0.0])
+def test_automatic_segments_lose_no_precision(pkg, dev, Hk, Hv, D, lens, decay):
+    """Segments move the state through the fp16-operand transitions P; with states
+    that decay slowly or not at all they stay as close to float64 as one pass.
+    (Measured over 1,700 to 16,000 tokens: both 2.2e-4 of the states at a decay of
+    0.02, 3.7e-4 to 4.0e-4 without; the two differ by at most 1.5 %, to either
+    side, so a factor of 1.05 is allowed.)"""
+    gen = torch.Generator().manual_seed(57)
+    q, k, v, g, beta = rule_inputs(gen, sum(lens), Hk, Hv, D)
+    g = g * decay
+    cu = torch.tensor(cu_of(lens), dtype=torch.int64)
+    h0 = torch.randn(len(lens), Hv, D, D, generator=gen) * 0.1
+    q, k, v, g, beta, h0 = (t.to(dev) for t in (q, k, v, g, beta, h0))
+    unit = lambda t: (t * (t.square().sum(-1, keepdim=True) + 1e-6).rsqrt()).repeat_interleave(Hv // Hk, 1)
+    qd, kd, vd, gd, bd = unit(q.double()) * D ** -0.5, unit(k.double()), v.double(), g.double().exp(), beta.double()
+    ro, rS = torch.empty_like(vd), h0.double()
+    for r in range(len(lens)):
+        S = rS[r]
+        for t in range(int(cu[r]), int(cu[r + 1])):
+            S = S * gd[t, :, None, None]
+            delta = (vd[t] - (S * kd[t, :, :, None]).sum(-2)) * bd[t, :, None]
+            S = S + kd[t, :, :, None] * delta[:, None, :]
+            ro[t] = (S * qd[t, :, :, None]).sum(-2)
+        rS[r] = S
+    rel = lambda x, y: float((x.double() - y).norm() / y.norm())
+    args = (q, k, v, g, beta, cu.to(dev), h0)
+    o_a, S_a = pkg.ops.chunk_gated_delta_rule_varlen(*args, cu_seqlens_cpu=cu)
+    o_1, S_1 = pkg.ops.chunk_gated_delta_rule_varlen(*args, cu_seqlens_cpu=cu, max_segments=1)
+    print(f"states {rel(S_a, rS):.3e} / one pass {rel(S_1, rS):.3e}, outputs {rel(o_a, ro):.3e} / {rel(o_1, ro):.3e}")
+    assert not torch.equal(S_a, S_1), "these lengths are cut"
+    assert rel(S_a, rS) <= 1.05 * rel(S_1, rS) and rel(o_a, ro) <= 1.05 * rel(o_1, ro)
+
+
 # empty sequences at the start, between others and at the end; lengths around a
 # chunk; the most sequences that the host's list holds, and one more
 @pytest.mark.parametrize("D,lens", [(128, [0, 1, 64, 0, 0, 65, 130, 3, 63, 128, 5, 200, 0]),
