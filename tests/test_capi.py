@@ -227,3 +227,15 @@ def test_column_part_gemm_validation_before_launch(pkg):
     for ends in ((40, 96), (64, 100), (96, 64), (64, 64), (8, 48, 64, 96)):
         assert call(ends, A=P) == _lib.GDN_ERR_INVALID_ARG, ends
     assert call((64, 96), lds=[32, 128, 128, 128, 128], A=P) == _lib.GDN_ERR_INVALID_ARG   # ld < part width
+
+
+def test_stream_handle_of_a_device_without_an_index(pkg, monkeypatch):
+    """torch.device("cuda") is torch's current device, as in torch's own calls."""
+    seen = []
+
+    def current_stream(device):
+        seen.append(device)
+        return type("Stream", (), {"cuda_stream": 7})
+
+    monkeypatch.setattr(torch.cuda, "current_stream", current_stream)
+    assert pkg._lib.stream_handle(torch.device("cuda")) == 7 and seen == [torch.device("cuda")]
