@@ -316,6 +316,9 @@ int gdn_recurrent_decode_fused(const uint16_t* q, int64_t sq_b, const uint16_t* 
  * gdn_conv_decode over the q and k channels followed by
  * gdn_recurrent_decode_fused.  The arguments are that entry point's, without
  * q and k; x is 16-byte aligned with a row stride that is a multiple of 8.
+ * With two value heads per key head it is the faster form below about 5120
+ * (row, value head) tiles; from there on the q/k channels' gdn_conv_decode
+ * followed by gdn_recurrent_decode_fused is.
  */
 int gdn_decode_step(const uint16_t* x, int64_t sx_row, uint16_t* conv_pool, int64_t cp_slot, int64_t cp_ch,
                     const uint16_t* conv_w, const uint16_t* a, const uint16_t* b, const void* A_log,
@@ -370,6 +373,10 @@ int gdn_state_tile_copy(const float* src, float* dst, int64_t slot_stride, const
  *   [gate_col + Hv, gate_col + 2 Hv) the a projection; from their bf16 values
  *   beta [M, Hv] bf16 and g [M, Hv] fp32 are also written, as gdn_g_beta
  *   computes them (fused_g_beta, qwen3_5.py:345-360).
+ * The order in which a row's K products are added may depend on M, N and K: calls
+ * of few tiles with K >= 1024 add four partial sums, all others in K's order, so
+ * a row's result in a small batch can differ in the last bit from the same row's
+ * in a larger one.
  */
 int gdn_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc, int M,
                   int N, int K, float* g, uint16_t* beta, const void* A_log, const void* dt_bias, int param_is_fp32,

@@ -2004,11 +2004,13 @@ __global__ __launch_bounds__(256) void seg_scan_kernel(ScanList sl, int Hv) {
 // S_{s+1}[:, block] = P_s S_s[:, block] + R_s[:, block], 32 products of
 // v_mfma_f32_16x16x4_f32.  Product (j, i) takes key 16 j + 4 g + i from lane
 // group g, so that a lane's A elements are eight float4 of one row of P_s: they
-// go straight from L2 (the 8 blocks of a head share one XCD's) to registers, the
-// next step's as soon as this one's are used.  S_s goes round through LDS, two
-// buffers, one barrier per step.  What bounds it: the latency of a step's chain
-// (LDS, 32 dependent products in two accumulators).  Seven steps at 16 heads: 27.4
-// us before (P_s staged through LDS, four waves of 64 products each).
+// go straight to registers, the next step's as soon as this one's are used (the 8
+// blocks of a head share an XCD's L2, into which the first of them brings P_s from
+// memory).  S_s goes round through LDS, two buffers, one barrier per step.  What
+// bounds it: those loads, one step ahead of their use: 3 us a step, where a step's
+// chain (LDS, 32 dependent products in two accumulators) takes about one.  Seven
+// steps at 16 heads: 21.4 us, 27.4 with P_s staged through LDS and four waves of 64
+// products each.
 __global__ __launch_bounds__(512) void seg_scan_mfma_kernel(ScanList sl, int Hv) {
   constexpr int D = 128;
   constexpr int CB = 16;

@@ -14,15 +14,19 @@
 // LDS read.
 //
 // Four kernels, chosen by gemm_launch:
-//   gemm_tn_pp_kernel    256 x 256 tiles, the last few as 128 x 128 quarters;
-//                        8 waves in two alternating groups, persistent (most
-//                        shapes with more than a few hundred rows)
+//   gemm_tn_pp_kernel    256 x 256 tiles, the last few as 128 x 128 quarters, or
+//                        128 x 128 blocks alone; 8 waves in two alternating
+//                        groups, persistent (most shapes with more than a few
+//                        hundred rows)
 //   gemm_tn_ring_kernel  16, 32 or 64 rows x 32 columns, K dealt to the waves,
 //                        a load ring per wave (few tiles: a decode out_proj)
 //   gemm_tn_deep_kernel  64 x 128 or 64 x 64, three or four LDS stages (a
 //                        decode in_proj)
 //   gemm_tn_kernel       the general one: 256 x 256 or 192 x 256 where K is an
-//                        odd multiple of 64, 64-row tiles where K is short
+//                        odd multiple of 64 or 192-row tiles run in one round,
+//                        64-row tiles where K is short
+// All but the ring kernel add a row's products in K's order, so they give the
+// same bits; the ring kernel adds four partial sums.
 //
 // gemm_tn_kernel: a workgroup of 4 waves (one per SIMD, one workgroup per CU)
 // computes a BM x BN tile of C, K in steps of 64.  Wave (wm, wn) owns rows BM /

@@ -802,7 +802,8 @@ namespace {
 // traffic, and recurrent_kernel, whose barriers drain each tile's loads before
 // its stores begin, moves it faster (256 x 16 tiles: 94.8 us against 96.1-98.7;
 // graph-replayed core of 127 x 16 tiles: 56.6 against 64.7 us for the three
-// launches that such batches took, 37 x 16 25.2 against 29.3)
+// launches that such batches took, 37 x 16 25.2 against 29.3).  Both kernels take
+// the same rows and give the same bits, so callers need not know the line.
 constexpr int64_t kStepTiles = 2048;
 
 // The checks that both entry points of the fused decode step share: float4

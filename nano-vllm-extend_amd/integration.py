@@ -35,8 +35,9 @@ With NANOVLLM_GDN_FUSED_DECODE=1 (the default) it replaces
 Qwen3_5GatedDeltaNet._gdn_padded (qwen3_5.py:967-1085) with one whose
 T == 1 branch runs ops.recurrent_decode_fused (gates, the conv with its
 roll, the in-place recurrent update and the gated norm self.norm in one
-kernel, after the q/k decode conv's own launch with more than two value heads
-per key head; the same results bit for bit); other T keep the original method.
+kernel, the q/k decode conv included with one value head per key head, and with
+two below ops.GROUPED_STEP_TILES (row, value head) tiles, else after that conv's
+own launch; the same results bit for bit); other T keep the original method.
 
 Both methods read the module's _USE_GDN_GBETA and _USE_CONV_TRITON (and the
 decode method _USE_GDN_INPLACE) on every call, as the reference's layer
@@ -109,8 +110,7 @@ def _fused_decode_method(mod, orig):
         proj = self.in_proj_qkv(x).reshape(-1, self.conv_dim)
         w = self.conv1d.weight.view(self.conv_dim, 4)
         kd = self.key_dim
-        # one or two value heads per key head: the q/k conv runs in the decode
-        # kernel too; else as its own launch first
+        # the q/k conv runs in the decode kernel too, or as its own launch first
         qk = None
         if not ops.one_launch_decode(n, self.num_k_heads, Hv):
             qk = ops.conv_decode_step(proj[:, :2 * kd], self.conv_cache[:, :2 * kd], ids, w[:2 * kd])

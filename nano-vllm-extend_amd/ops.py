@@ -594,7 +594,9 @@ def recurrent_gdn_inplace(q, k, v, g, beta, s_pool, ids):
 # workgroup.  With fewer the head's columns may be split over workgroups: in the
 # multi-token kernel that changes the summation order of S^T k, so its
 # whole-head and split runs differ in the last bits; one-token steps add in one
-# order at every split.
+# order at every split.  (Also the line below which the one-launch step takes
+# only the rows that the q/k conv's launch, which ran there before it, takes; the
+# library's own line between its two one-launch kernels is a matter of speed.)
 WHOLE_HEAD_TILES = 2048
 
 

@@ -110,6 +110,17 @@ def test_gemm_kernel_choice(pkg, dev, M, N, K, Hv):
     test_gemm_kernel_edges(pkg, dev, M, N, K, Hv)
 
 
+def test_gemm_rows_do_not_depend_on_the_batch(pkg, dev):
+    """64 x 128 tiles, 128 x 128 blocks, 192-row tiles and 256 x 256 tiles with a
+    tail add a row's products in the same order: the same bits for the same rows."""
+    gen = torch.Generator().manual_seed(8)
+    x = torch.randn(2500, 1280, generator=gen).to(BF16).to(dev)
+    w = (torch.randn(8224, 1280, generator=gen) / 36).to(BF16).to(dev)
+    c = pkg.ops.linear(x, w)
+    for M in (129, 300, 900):
+        assert torch.equal(pkg.ops.linear(x[:M], w).view(torch.int16), c[:M].view(torch.int16)), M
+
+
 @pytest.mark.parametrize("pad,off", [(40, 8), (41, 3)])
 def test_gemm_strided_operands_and_out(pkg, dev, pad, off):
     """Row strides larger than K (views of wider buffers) and an output view;
