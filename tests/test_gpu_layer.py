@@ -503,3 +503,28 @@ def test_split_state_pass_equals_one_stream(pkg, dev):
     assert torch.equal(o1.view(torch.int16), o2.view(torch.int16)), "outputs differ"
     assert torch.equal(c1.view(torch.int16), c2.view(torch.int16)), "conv pool differs"
     assert torch.equal(s1, s2), "state pool differs"
+
+
+def test_split_state_pass_with_segments(pkg, dev):
+    """The split over two streams where both sides are cut into segments (slowly
+    decaying states): the one-stream results bit for bit, pools included."""
+    lens, Hk, Hv, D = [49675, 1893, 573], 16, 16, 128
+    split = pkg.gdn_layer.late_split(lens, Hv)
+    assert split is not None and split[0] == [True, False, False]
+    gen = torch.Generator(device=dev).manual_seed(58)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device=dev)
+    n, N, C = len(lens), sum(lens), 2 * Hk * D + Hv * D
+    mixed, z, a, b = (rand(N, w).to(BF16) for w in (C, Hv * D, Hv, Hv))
+    conv_w, norm_w = (rand(C, 4) * 0.5).to(BF16), (1 + 0.02 * rand(D)).to(BF16)
+    A_log, dt_bias = (rand(Hv) * 0.3 - 4).to(BF16), rand(Hv).to(BF16)
+    conv0, s0 = rand(n, C, 3).to(BF16), rand(n, Hv, D, D) * 0.1
+    outs = []
+    for on in (False, True):
+        core = _core(pkg, dev, Hk, Hv, D, conv_w, A_log, dt_bias, norm_w, split_state=on)
+        cp, sp = conv0.clone(), s0.clone()
+        outs.append((core.prefill_varlen(mixed, z, b, a, lens, torch.arange(n, device=dev), cp, sp), cp, sp))
+        torch.cuda.synchronize()
+    (o1, c1, s1), (o2, c2, s2) = outs
+    assert torch.equal(o1.view(torch.int16), o2.view(torch.int16)), "outputs differ"
+    assert torch.equal(c1.view(torch.int16), c2.view(torch.int16)), "conv pool differs"
+    assert torch.equal(s1, s2), "state pool differs"
