@@ -30,17 +30,13 @@ def _ref(a, w):
     return a.float() @ w.float().t(), a.float().abs() @ w.float().abs().t()
 
 
-# The tile is 256 x 256, or 192 x 256 when ceil(tiles / 256 CUs) x rows is
-# smaller with it, or 64 x 128 when fewer than 128 tiles of 256 x 256 would
-# run, or 64 x 64 when fewer than 128 of 64 x 128 would.  The 64-row tiles run
-# the deeper load pipeline (gemm_tn_deep_kernel) when K >= 1024.  64 x 64:
-# (256, 256), (300, 200); deep: (1, 8224), (17, 2048), (256, 2048) (the decode
-# out_proj), (100, 2000, 1088) (17 steps: a partial last round of stages);
-# 64 x 128: (1000, 2080), (4111, 333); deep: (256, 8224) (the decode in_proj),
-# (300, 8224, 1024) (16 steps, ragged rows);
-# 192 x 256: (17000, 2048) = 712 tiles of 192 rows (3 waves) against 536 of 256
-# (3 waves); 256 x 256: (8190, 2047) is exactly 256 tiles of 256 rows (344 of
-# 192) and (17000, 8224) ties at 9 waves.
+# 64 x 64 tiles: (256, 256), (300, 200); with the deeper load pipeline (K >= 1024):
+# (1, 8224); 64 x 128: (1000, 2080), (4111, 333); deeper: (300, 8224, 1024) (16
+# steps, ragged rows).  The ring kernel: (17, 2048), (256, 2048) (the decode
+# out_proj), (100, 2000, 1088) (17 steps dealt to four waves).  The 8-wave kernel:
+# (256, 8224) (the decode in_proj, as 130 blocks of 128 x 128), (17000, 2048) (512
+# whole tiles and 24 as quarters), (8190, 2047) (one exact round), (17000, 8224)
+# (2211 whole tiles).
 @pytest.mark.parametrize("M,N,K", [(256, 256, 64), (300, 200, 128), (1, 8224, 2048), (17, 2048, 2048), (256, 2048, 2048),
                                    (100, 2000, 1088), (1000, 2080, 512), (4111, 333, 192), (256, 8224, 2048),
                                    (300, 8224, 1024), (17000, 2048, 256), (8190, 2047, 128), (17000, 8224, 128)])
@@ -53,11 +49,11 @@ def test_gemm_against_fp32_matmul(pkg, dev, M, N, K):
     _check(c, ref, sc, f"gemm {M}x{N}x{K}")
 
 
-# The 8-wave kernel's quarters alone (128 x 128; K of 2, 4 and 6 steps, ragged
-# rows and columns, an empty quarter past M), behind whole tiles, and whole tiles
-# of an uneven last round; its K restriction (192: gemm_tn_kernel at 256 and 192
-# rows); the ring kernel at 16, 32 and 64 rows with 16, 17 and 33 steps (dealt to
-# four waves: uneven).  Hv > 0: the columns go to four parts with gate outputs
+# 64 x 128 tiles of a short K with ragged rows and columns (the first three); whole
+# tiles of the 8-wave kernel with a tail of quarters, an empty one past M, and of an
+# uneven round; its K restriction (192: gemm_tn_kernel at 256 and 192 rows); the
+# ring kernel at 16 and 32 rows, and 64 x 64 tiles, with 16, 17 and 33 steps (dealt
+# to four waves: uneven).  Hv > 0: the columns go to four parts with gate outputs
 # (b and a the last 2 Hv columns).
 @pytest.mark.parametrize("M,N,K,Hv", [(1949, 2048, 128, 0), (1100, 4000, 256, 16), (1153, 2072, 384, 4),
                                       (4100, 4008, 384, 4), (4500, 3000, 256, 0), (8190, 2047, 192, 0),
@@ -177,7 +173,8 @@ def test_in_proj_column_parts_equal_one_output(pkg, dev, M, with_gates, layout):
     """gdn_gemm_bf16_cols (the layer's in_proj into separate qkv, z, b and a
     tensors): every part bit-equal to the same columns of the one-output GEMM,
     and the gate outputs too, for each tile shape (M = 64: 64 x 64 tiles with
-    the deeper pipeline, 100: 64 x 128, 777: 192 x 256, 1790: 256 x 256)."""
+    the deeper pipeline, 100: 64 x 128, 777: 256 x 256, 1790: 256 x 256 with a
+    tail of quarters)."""
     gen = torch.Generator().manual_seed(7)
     Hk, Hv = 16, 32
     D, hidden = 128, 2048
