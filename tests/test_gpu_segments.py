@@ -98,7 +98,7 @@ def test_segmented_fused_prefill(pkg, dev):
     assert torch.equal(c6.view(torch.int16), c1.view(torch.int16)), "conv states"
 
 
-# the automatic plan: one pass (a short sequence), the fewest chunks it cuts, a
+# the automatic plan: one pass (a short sequence), 30 chunks in segments, a
 # second sequence cut in two beside one that is not, and every sequence cut
 @pytest.mark.parametrize("lens", [[300], [1900], [4000, 1500, 70], [2600, 2500]], ids=str)
 def test_automatic_segments(pkg, dev, lens):
