@@ -99,7 +99,7 @@ def test_segmented_fused_prefill(pkg, dev):
 
 
 # the automatic plan: one pass (a short sequence), 30 chunks in segments, a
-# second sequence cut in two beside one that is not, and every sequence cut
+# second sequence cut in fewer beside one that is not, and every sequence cut
 @pytest.mark.parametrize("lens", [[300], [1900], [4000, 1500, 70], [2600, 2500]], ids=str)
 def test_automatic_segments(pkg, dev, lens):
     """Slowly decaying states (g of a few hundredths), so that the scan's
